@@ -365,15 +365,15 @@ void build_gtab(const Archive& X, uint8_t* out) {
             ent[j] = e;
         }
     }
-    // literal pairs (the vector decoder's two-literal step): from the LIT2 rows just written
+    // literal entries (the wave decoder's triple step): from the LIT2 rows just written
     uint32_t* pr = (uint32_t*)(out + pvc::PAIR_OFF);
     const uint16_t* l2 = t + pvc::row_of(pvc::C_LIT2);
     for (int r = 0; r < 16; r++)
         for (int l = 0; l < 16; l++) {
             const int s1 = l >> 2, s2 = l & 3, r1 = (r & 3) * 4 + s1;
             const uint16_t* a = l2 + r * pvc::SMALL_ROW; const uint16_t* b = l2 + r1 * pvc::SMALL_ROW;
-            pr[2 * (16 * r + l)] = a[s1] | (uint32_t)(a[s1 + 1] - a[s1] - pvc::M) << 16;
-            pr[2 * (16 * r + l) + 1] = b[s2] | (uint32_t)(b[s2 + 1] - b[s2] - pvc::M) << 16;
+            pr[2 * (16 * r + l)] = pvc::pair_entry(a[s1], a[s1 + 1]);
+            pr[2 * (16 * r + l) + 1] = pvc::pair_entry(b[s2], b[s2 + 1]);
         }
 }
 

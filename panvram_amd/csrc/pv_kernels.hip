@@ -221,13 +221,89 @@ __device__ __forceinline__ uint32_t sym_small(Dec& d, const Small& R, uint32_t r
     return s;
 }
 // Literal triples. Lane l stands for the symbol triple (s1, s2, s3) = (l >> 4, (l >> 2) & 3, l & 3) and holds, for each
-// of the 16 order-2 literal contexts r, (lo | (freq - 4096) << 16) of s1 in context r (low half of AB[r]) and of s2 in
-// the context after s1 (high half), and (C) of s3 in the context after s1 s2, which does not depend on r. All come from
-// the model table's pair section, loaded on a block's first long literal run; AB is indexed by the wave-uniform
-// context, which the compiler turns into one indexed move of a register pair.
-typedef uint64_t v16ul __attribute__((ext_vector_type(16)));
-// count of leading zeros (32 for 0; only lanes whose hypothesis fails can see 0)
-__device__ __forceinline__ uint32_t ffbh(uint32_t v) { uint32_t r; asm("v_ffbh_u32 %0, %1" : "=v"(r) : "v"(v)); return r; }
+// of the 16 order-2 literal contexts r, the entry of s1 in context r (A[r]) and of s2 in the context after s1 (B[r]), and
+// that of s3 in the context after s1 s2 (C), which does not depend on r: lo << 4 | freq << 20 each, from the model
+// table's pair section, loaded on a block's first long literal run.
+//
+// literal_windows decodes up to LIT_RUN windows of three triples (nine literals each) in one assembly loop. Each lane
+// decodes its triple from the current state as if it were right; the lanes whose three slots fall in their symbols'
+// ranges stay active (v_cmpx narrows exec), so that the one left holds the new state, and its number the next context.
+//
+//  - A lane's state is the pair v[96:97]: the high word is x << 4 | the next 4 payload bits, the low word the 32 bits
+//    after those, its last bit set to mark their end. With the 12-bit slot in bits 4-15 and x >> 12 in the high half
+//    word, v_sub (half words) gives the slot's place z in the symbol's range, z < freq << 4 is the range check and
+//    v_mad_u32_u16 on the high halves the decode step; one 64-bit shift by 0 or 8 renormalises, and moves the window.
+//    One byte is enough for a symbol of frequency 16 or more (x >= 2^16 before it); rarer symbols, and a context's only
+//    one (its frequency does not fit 12 bits), have entries of frequency 0, which no slot is in.
+//  - A window takes at most 24 payload bits. How many it took is the place of the end mark; the next window's low word
+//    is lane (bytes taken) of `words`, whose lane i holds the 32 bits from 4 bits past payload byte i on. 32 bits or
+//    more leave no mark, a triple that no lane has right (an N or escape literal among it) no active lane: s_ff1 then
+//    gives -1, the sign bit of `fail` is set and the loop leaves after that window; the caller decodes again from the
+//    run's start with as many windows as were good, and the nine literals that were not on the general path.
+//  - The index register (the context, which picks A[r] and B[r]) is set per triple around two moves.
+//
+// What bounds it is one wave's issue: 4 clocks for a 4-byte instruction, 5.6-6.4 for an 8-byte one, and up to 16 more
+// for a scalar instruction within four vector ones of a vector write to SGPRs, vcc or exec, dependent or not; hence the
+// order below (s_ff1 after the two lane reads; mad before cmpx, except in the third literal, whose check the
+// select reads first). Measured on one wave, 4,005 literals (shader clocks a literal): 98.3 with the triple step in C++
+// (63 instructions a triple: two 64-bit shifts per renormalisation, masks in SGPRs, byte counts packed into the
+// state), 82.9 with this step and C++ around three triples, 65.8 with the whole loop in assembly and the shift
+// from leading zeros, 64.5 with it from a compare, 61.1 with v_readfirstlane under the narrowed exec, 59.4 with the
+// scalar work ordered as it is; a window's bookkeeping moved into the next triple's first literal 59.3. In the kernels:
+// front_kernel of sample(1024, 8192) 168 -> 120 us (mean of 13 calls), the longest q16k block 715 -> 450 us.
+typedef uint32_t v16u __attribute__((ext_vector_type(16)));
+constexpr uint32_t LIT_WIN = 9, LIT_RUN = 21;      // literals per window; windows per run (3 bytes each: words' 64 lanes)
+#define PV_LIT_STEP(src, e) \
+    "v_sub_u32_sdwa %[z], " src ", " e " dst_sel:DWORD dst_unused:UNUSED_PAD src0_sel:WORD_0 src1_sel:WORD_0\n"
+#define PV_LIT_MAD(src, e) "v_mad_u32_u16 v97, " src ", " e ", %[z] op_sel:[1,1,0,0]\n"
+#define PV_LIT_CHECK(e) "v_cmpx_lt_u32_sdwa vcc, %[z], " e " src0_sel:DWORD src1_sel:WORD_1\n"
+#define PV_LIT_NORM "v_cmp_gt_u32 vcc, %[low], v97\n" "v_cndmask_b32 %[z], 0, %[eight], vcc\n" "v_lshlrev_b64 v[96:97], %[z], v[96:97]\n"
+// the context's entries (acc's low four bits; idx: the register they are put in), then the triple and its select
+#define PV_LIT_TRIPLE(idx) \
+    "s_and_b32 " idx ", %[acc], 15\n" "s_set_gpr_idx_on " idx ", gpr_idx(SRC0)\n" "v_mov_b32 %[a], v64\n" "v_mov_b32 %[b], v80\n" \
+    "s_set_gpr_idx_off\n" "v_mov_b32 v96, %[lo]\n" \
+    PV_LIT_STEP("%[y]", "%[a]") PV_LIT_MAD("%[y]", "%[a]") PV_LIT_CHECK("%[a]") PV_LIT_NORM \
+    PV_LIT_STEP("v97", "%[b]") PV_LIT_MAD("v97", "%[b]") PV_LIT_CHECK("%[b]") PV_LIT_NORM \
+    PV_LIT_STEP("v97", "%[c]") PV_LIT_CHECK("%[c]") PV_LIT_MAD("v97", "%[c]") PV_LIT_NORM \
+    "s_nop 0\n" "v_readfirstlane_b32 %[lo], v96\n" "v_readfirstlane_b32 %[y], v97\n" "s_ff1_i32_b64 %[t], exec\n" \
+    "s_lshl_b32 %[acc], %[acc], 6\n" "s_mov_b64 exec, %[ex]\n" "s_or_b32 %[acc], %[acc], %[t]\n"
+// y: x << 4 | the next 4 payload bits; r: the context; words: as above; n: windows (1 .. LIT_RUN), all lanes the same.
+// Returns in lane i of `lits` window i's context and literals (4 + 18 bits, the first literal's highest), in y, r and
+// bits the state after the last window, in n the windows done, the last of them not good when fail is negative.
+__device__ __forceinline__ void literal_windows(uint32_t& y, uint32_t& r, uint32_t& n, uint32_t& bits, int32_t& fail, uint32_t& lits,
+                                                uint32_t words, const v16u& A, const v16u& B, uint32_t C) {
+    uint32_t yy = rfl(y), acc = rfl(r), lo = rdl(words, 0), k = 0, P = 0, t, i, z, a, b, m; int32_t f; uint64_t ex;
+    const uint32_t end = rfl(n);
+    asm volatile(
+        "s_mov_b64 %[ex], exec\n"
+        "s_mov_b32 %[m], m0\n"
+        ".Lliteral%=:\n"
+        PV_LIT_TRIPLE("%[acc]") PV_LIT_TRIPLE("%[i]") PV_LIT_TRIPLE("%[i]")
+        "s_mov_b32 m0, %[k]\n"
+        "s_ff1_i32_b32 %[t], %[lo]\n"
+        "s_add_u32 %[k], %[k], 1\n"
+        "s_add_u32 %[P], %[P], %[t]\n"
+        "s_or_b32 %[f], %[acc], %[t]\n"
+        "s_lshr_b32 %[i], %[P], 3\n"
+        "s_sub_u32 %[t], %[k], %[end]\n"
+        "s_andn2_b32 %[t], %[t], %[f]\n"
+        "s_cmp_lt_i32 %[t], 0\n"
+        "v_writelane_b32 %[lits], %[acc], m0\n"
+        "v_readlane_b32 %[lo], %[words], %[i]\n"
+        "s_cbranch_scc1 .Lliteral%=\n"
+        "s_mov_b32 m0, %[m]\n"
+        "s_nop 1\n"
+        : [y] "+&s"(yy), [lo] "+&s"(lo), [acc] "+&s"(acc), [k] "+&s"(k), [P] "+&s"(P), [lits] "+&v"(lits), [t] "=&s"(t), [i] "=&s"(i), [f] "=&s"(f),
+          [ex] "=&s"(ex), [m] "=&s"(m), [z] "=&v"(z), [a] "=&v"(a), [b] "=&v"(b)
+        : "{v[64:79]}"(A), "{v[80:95]}"(B), [c] "v"(C), [words] "v"(words), [end] "s"(end), [low] "s"(0x100000u), [eight] "v"(8u)
+        : "v96", "v97", "vcc", "scc");
+    y = rfl(yy); r = rfl(acc) & 15; n = rfl(k); bits = rfl(P); fail = (int32_t)rfl((uint32_t)f);
+}
+#undef PV_LIT_STEP
+#undef PV_LIT_MAD
+#undef PV_LIT_CHECK
+#undef PV_LIT_NORM
+#undef PV_LIT_TRIPLE
 
 // 104-letter context: lane l compares cum[l+1] and cum[l+65] (LDS); the symbol is the count of boundaries <= slot
 template <int Q, bool G> __device__ __forceinline__ uint32_t sym_big(const DecMem<Q, G>& M, Dec& d, uint32_t row) {
@@ -397,7 +473,7 @@ template <int Q, bool G> __device__ __forceinline__ int decode_block(const DecMe
     Cache C; C.init(c0, dir0);
     int prevk = -1; uint32_t o = 0; int nops = 0;
     LitAcc lit; lit.v = 0; lit.k = 0; lit.base = 0;
-    v16ul AB; uint32_t PC = 0; bool pready = false;      // literal-triple tables, loaded on the first long run
+    v16u A, B; uint32_t PC = 0; bool pready = false;     // literal-triple entries, loaded on the first long run
     constexpr uint32_t ACGTN = 'A' | ('C' << 8) | ('G' << 16) | ('T' << 24);
     while (o < blen) {
         o = rfl(o); prevk = (int)rfl((uint32_t)prevk); nops = (int)rfl((uint32_t)nops);
@@ -435,85 +511,69 @@ template <int Q, bool G> __device__ __forceinline__ int decode_block(const DecMe
                     lit.put(S, byte); lit.flush(S);
                     r = s < 4 ? s : 0; j = 1;
                 }
-                // Triple steps: every lane decodes its triple (s1, s2, s3) from the current state as if it were right -
-                // symbol step, renormalisation (its byte count from the leading zeros, the bytes from the big-endian
-                // window V of buffered payload), and so on for s2 and s3, each in the context its predecessors lead
-                // to - and checks that all three slots fall in its symbols' ranges. Exactly one lane passes when the
-                // three literals are A/C/G/T; its index holds the next context and v_readlane takes its state and byte
-                // count. A group of five triples commits when all found a lane and the bytes they read were buffered
-                // and inside the payload; otherwise its fifteen literals are decoded again on the general path (the
-                // state is untouched).
-                constexpr uint32_t G3 = 5;                   // triples per commit: 15 literals, 30 bits of codes
-                if (j + 3 * G3 <= (uint32_t)ll && !pready) {
+                // Triple steps (literal_windows), nine literals at a time; the nine that a window did not get right - an N
+                // or escape literal among them, a rare symbol, more than 24 payload bits - on the general path.
+                if (j + LIT_WIN <= (uint32_t)ll && !pready) {
                     // lane l = 16 s1 + 4 s2 + s3: s1 in the run's context r and s2 in the context after s1 from the pair
                     // section's entry (r, l >> 2); s3 in context (l >> 2) = 4 s1 + s2, the pair section's first entry
                     // of that context for symbol l & 3
                     const uint2* src = (const uint2*)(gtab + pvc::PAIR_OFF);
                     const uint32_t pl = lane_id() >> 2;
 #pragma unroll
-                    for (int k = 0; k < 16; k++) { const uint2 e = src[16 * k + pl]; AB[k] = (uint64_t)e.x | ((uint64_t)e.y << 32); }
+                    for (int k = 0; k < 16; k++) { const uint2 e = src[16 * k + pl]; A[k] = e.x; B[k] = e.y; }
                     PC = src[16 * pl + 4 * (lane_id() & 3)].x;
                     pready = true;
                 }
-                while (j + 3 * G3 <= (uint32_t)ll) {
-                    // groups on the triple path while they commit; a group that does not (an N or escape literal
-                    // among its fifteen, or bytes past the buffer) leaves this loop for the general path below. The
-                    // loop has one exit and no early return, so that the compiler keeps it tight (merged into the
-                    // decoder's outer loop it took 112 instead of 100 clocks per literal).
-                    bool stalled = false;
-                    do {
-                        if (d.cnt <= 4) refill(d);
-                        uint64_t V = __builtin_bswap64(d.buf);       // buffered bytes, first in the top byte (zeros past cnt)
-                        uint32_t x = d.x, bits = 0, orL = 0, acc = 0, rr = rfl(r);
-#pragma unroll
-                        for (uint32_t u = 0; u < G3; u++) {
-                            const uint64_t ab = AB[rr & 15];
-                            const uint32_t a = (uint32_t)ab, b = (uint32_t)(ab >> 32);
-                            // With F = freq - 4096: F (x >> 12) + (x - lo) = freq (x >> 12) + (x & 4095) - lo, the decode step,
-                            // and x's slot is in [lo, lo + freq) iff ((x - lo) & 4095) - 4096 < F (lo + freq <= 4096).
-                            // Renormalisation: the state's leading zeros give the payload bits it takes (0, 8 or 16), and a
-                            // 64-bit shift of (state, next payload word) by that many moves them in.
-                            const int32_t Fa = (int32_t)a >> 16;
-                            const uint32_t u1 = x - (a & 0xFFFF);
-                            const uint64_t m1 = __ballot((int32_t)(u1 | 0xFFFFF000u) < Fa);
-                            const uint32_t y = (uint32_t)(__mul24(Fa, (int32_t)(x >> pvc::PROB_BITS)) + (int32_t)u1);
-                            const uint32_t s1 = (ffbh(y) - 8) & 24;
-                            const uint32_t y1 = (uint32_t)(((((uint64_t)y << 32) | (uint32_t)(V >> 32)) << s1) >> 32);
-                            const uint64_t Vb = V << s1;                              // window after those bytes
-                            const int32_t Fb = (int32_t)b >> 16;
-                            const uint32_t u2 = y1 - (b & 0xFFFF);
-                            const uint64_t m2 = __ballot((int32_t)(u2 | 0xFFFFF000u) < Fb);
-                            const uint32_t z = (uint32_t)(__mul24(Fb, (int32_t)(y1 >> pvc::PROB_BITS)) + (int32_t)u2);
-                            const uint32_t s2 = (ffbh(z) - 8) & 24;
-                            const uint32_t z1 = (uint32_t)(((((uint64_t)z << 32) | (uint32_t)(Vb >> 32)) << s2) >> 32);
-                            const uint64_t Vc = Vb << s2;
-                            const int32_t Fc = (int32_t)PC >> 16;
-                            const uint32_t u3 = z1 - (PC & 0xFFFF);
-                            const uint64_t m3 = __ballot((int32_t)(u3 | 0xFFFFF000u) < Fc);
-                            const uint32_t q = (uint32_t)(__mul24(Fc, (int32_t)(z1 >> pvc::PROB_BITS)) + (int32_t)u3);
-                            const uint32_t s3 = (ffbh(q) - 8) & 24;
-                            const uint32_t q1 = (uint32_t)(((((uint64_t)q << 32) | (uint32_t)(Vc >> 32)) << s3) >> 32);
-                            const uint32_t res = q1 | ((s1 + s2 + s3) << 24);          // state | payload bits read
-                            uint32_t L;
-                            asm volatile("s_ff1_i32_b64 %0, %1" : "=s"(L) : "s"(m1 & m2 & m3));   // -1: no lane
-                            const uint32_t pick = rdl(res, L);
-                            x = pick & 0xFFFFFF;
-                            const uint32_t sb = pick >> 24;
-                            V <<= sb; bits += sb;
-                            orL |= L; acc = (acc << 6) + L;
-                            rr = L;
+                // Payload words for literal_windows: lane i those from byte p + i (w0) and p + 64 + i (w1) on (reads past
+                // the payload land in the pool's padding, and what they give is never taken: p > n fails the block as
+                // the byte that is not there would on the general path)
+                auto words = [&](uint32_t at, uint32_t& top) -> uint32_t {
+                    uint64_t w;
+                    __builtin_memcpy(&w, d.g + at + lane_id(), 8);
+                    w = __builtin_bswap64(w);
+                    top = (uint32_t)(w >> 60);
+                    return (uint32_t)(w >> 28) | 1u;
+                };
+                uint32_t y = 0, w0 = 0, w1 = 0, skip, cap = 0;       // cap: the windows the next run may take
+                bool fresh = true;                                    // y, w0, w1 do not hold the state in d
+                while (j + LIT_WIN <= (uint32_t)ll) {
+                    j = rfl(j);
+                    if (fresh && d.x >= pvc::RANS_L) {               // (below it only in a corrupt payload)
+                        w0 = words(d.p, skip);
+                        y = (d.x << 4) | rfl(skip);
+                        w1 = words(d.p + 64, skip);
+                        cap = LIT_RUN; fresh = false;
+                    }
+                    if (rfl(cap)) {
+                        uint32_t y1 = y, r1 = r, n = min(((uint32_t)ll - j) / LIT_WIN, cap), bits = 0, lits = 0; int32_t fail;
+                        literal_windows(y1, r1, n, bits, fail, lits, w0, A, B, PC);
+                        if (fail < 0) { cap = n - 1; if (cap) continue; }        // again, as far as it was good
+                        else {
+                            const uint32_t used = bits >> 3, m = n * LIT_WIN;
+                            d.p += used; d.x = y1 >> 4; y = y1; r = r1;
+                            if (d.p > d.n) return -1;
+                            // window i's literals from lane i: its t-th from bits 2 (8 - t) up
+                            for (uint32_t i0 = 0; i0 < m; i0 += WAVE) {
+                                const uint32_t i = i0 + lane_id(), wi = (i * 7282u) >> 16, t = i - 9 * wi;      // i / 9, i % 9
+                                const uint32_t v = (uint32_t)__shfl((int)lits, (int)wi);
+                                if (i < m) blk_put(S, o + j + i, (uint8_t)(ACGTN >> (8 * ((v >> (2 * (8 - t))) & 3))));
+                            }
+                            j += m;
+                            d.buf = 0; d.cnt = 0; d.q = d.p;
+                            if (cap < LIT_RUN && n == cap) cap = 0;              // the next window is the one not good
+                            else {
+                                // the words from the new place on: w0's and w1's lanes moved down by the bytes taken
+                                const uint32_t e = lane_id() + used;
+                                const uint32_t u0 = (uint32_t)__shfl((int)w0, (int)(e & 63)), u1 = (uint32_t)__shfl((int)w1, (int)(e & 63));
+                                w0 = e < WAVE ? u0 : u1;
+                                w1 = words(d.p + 64, skip);
+                                continue;
+                            }
+                            if (j + LIT_WIN > (uint32_t)ll) break;
                         }
-                        const uint32_t used = bits >> 3;
-                        // a triple with no lane (L = -1), or more bytes than buffered or left in the payload: the sign bits
-                        // of the differences (all small), on the scalar unit
-                        if ((orL >> 6) | ((d.cnt - used) >> 31) | ((d.n - d.p - used) >> 31)) { stalled = true; break; }
-                        d.x = x; d.buf = used < 8 ? d.buf >> (8 * used) : 0; d.cnt -= used; d.p += used; r = rr & 15;
-                        if (lane_id() < 3 * G3) blk_put(S, o + j + lane_id(), (uint8_t)(ACGTN >> (8 * ((acc >> (2 * (3 * G3 - 1 - lane_id()))) & 3))));
-                        j += 3 * G3;
-                    } while (j + 3 * G3 <= (uint32_t)ll);
-                    if (!stalled) break;
+                    }
                     lit.base = o + j;
-                    for (uint32_t u = 0; u < 3 * G3; u++, j++) {
+                    for (uint32_t u = 0; u < LIT_WIN; u++, j++) {
                         const uint32_t s = sym_small(d, SR, SR_LIT2 + r);
                         if (d.bad) return -1;
                         uint32_t byte = s < 4 ? (ACGTN >> (8 * s)) & 0xFF : 'N';
@@ -522,6 +582,7 @@ template <int Q, bool G> __device__ __forceinline__ int decode_block(const DecMe
                         r = rfl(((r * 4) + (s < 4 ? s : 0)) & 15);
                     }
                     lit.flush(S);
+                    fresh = true; cap = 0;
                 }
                 lit.base = o + j;
                 for (; j < (uint32_t)ll; j++) {
@@ -1002,7 +1063,7 @@ __device__ __forceinline__ v4u lds16(const uint32_t* a, uint32_t so) {
 template <int Q, bool DEC, class LS>
 __device__ __forceinline__ void process_slot(LS& S, const pv_dev_cohort& D, const SlotHdr& H, uint32_t state, const uint8_t* slot_pre,
                                              uint2 op0, const uint8_t* hs, uint32_t hnops, uint64_t w, uint32_t W, bool rc, int tokens,
-                                             int apply_case, void* out, const int64_t* ids, int* status);
+                                             int apply_case, void* out, const int64_t* ids, int* status, bool urgent);
 
 // The heavy list entry a heavy wave took t-th: slot_kernel's long ones from the front, then its short ones from the back
 __device__ __forceinline__ uint32_t entry_at(const HeavyList& HL, uint32_t nbig, uint32_t t) { return t < nbig ? t : HL.cap - 1u - (t - nbig); }
@@ -1031,9 +1092,10 @@ __device__ __forceinline__ bool entry_slot(const pv_dev_cohort& D, const int64_t
     return slot_at<Q>(D, a, s0, W, j, H) && rfl(H.state) == SLOT_WAVE;
 }
 
-// The wave decoder's decode of a slot's block into heavy area hs, in global memory (no LDS), at raised issue priority
-// for a long payload: the record {HEAVY_DONE, ops} or {HEAVY_FAILED, 0}, the copy ops and the block with its literals.
-template <int Q>
+// The wave decoder's decode of a slot's block into heavy area hs, in global memory (no LDS), in a small call (SMALL) at
+// raised issue priority for a long payload: the record {HEAVY_DONE, ops} or {HEAVY_FAILED, 0}, the copy ops and the block
+// with its literals. A large call's light lanes and replay take longer than its longest chain, which runs beside them.
+template <int Q, bool SMALL>
 __device__ __forceinline__ void decode_to_area(const pv_dev_cohort& D, const SlotHdr& H, uint8_t* hs) {
     const uint32_t l = lane_id();
     int nops = -1;
@@ -1066,7 +1128,7 @@ __device__ __forceinline__ void decode_to_area(const pv_dev_cohort& D, const Slo
     if (plen >= 3) {
         refill(d);
         d.x = (uint32_t)(d.buf & 0xFFFFFF); d.buf >>= 24; d.cnt -= 3; d.p = 3;
-        if (plen > HEAVY_PAY) __builtin_amdgcn_s_setprio(3);
+        if (SMALL && plen > HEAVY_PAY) __builtin_amdgcn_s_setprio(3);
         nops = (int)rfl((uint32_t)decode_block(M, OP, d, SR, gtab, R, blen, stv >> 1, (uint32_t)(stv & 1)));
         __builtin_amdgcn_s_setprio(0);
     }
@@ -1081,8 +1143,8 @@ __device__ __forceinline__ void decode_to_area(const pv_dev_cohort& D, const Slo
 }
 
 // A wave of heavy_kernel: wave k decodes the heavy list's k-th entry in take order (entry_at: the long ones first, then
-// the short ones) into heavy area k with the wave decoder, in global memory, at raised issue priority for a long
-// payload; the entry's done word then names the area. The grid has one wave per area, so each wave has at most one
+// the short ones) into heavy area k with the wave decoder, in global memory; the entry's done word then names the
+// area. The grid has one wave per area, so each wave has at most one
 // entry: the waves past the list's length (most of them) leave after reading its two counts, and entries past the area
 // count are left to spill_kernel. The list is final when the kernel starts (slot_kernel wrote it), so no wave waits.
 // Returns the slot it decoded, -1 past the list, -2 for an entry of another call (not reached).
@@ -1097,7 +1159,7 @@ __device__ __forceinline__ int64_t heavy_decode(const pv_dev_cohort& D, const in
     if ((uint32_t)(e >> 32) != HL.epoch) return -2;  // (not reached) windows_kernel reports the slot as status bit 4
     uint64_t w; bool rc; SlotHdr H;
     uint8_t* hs = HL.area + (uint64_t)t * Heavy<Q>::BYTES;
-    if (entry_slot<Q>(D, wasm, wstart, nullptr, W, bpw, X, (uint32_t)e, w, rc, H)) decode_to_area<Q>(D, H, hs);
+    if (entry_slot<Q>(D, wasm, wstart, nullptr, W, bpw, X, (uint32_t)e, w, rc, H)) decode_to_area<Q, false>(D, H, hs);
     else *(uint2*)hs = make_uint2(HEAVY_FAILED, 0u);
     HL.done[i] = (uint64_t)HL.epoch | ((uint64_t)t << 32);
     return (int64_t)(uint32_t)e;
@@ -1129,7 +1191,7 @@ __device__ __forceinline__ void whole_worker(Lds<Q>& S, const pv_dev_cohort& D, 
         *bits = 0;                                     // the slot's status bits, in LDS (process_slot ors into them)
         __syncthreads();
         if (entry_slot<Q>(D, wasm, wstart, rcm, W, bpw, X, (uint32_t)e, w, rc, H))
-            process_slot<Q, true>(S, D, H, SLOT_WAVE, nullptr, make_uint2(0, 0), nullptr, 0, w, W, rc, tokens, apply_case, out, ids, bits);
+            process_slot<Q, true>(S, D, H, SLOT_WAVE, nullptr, make_uint2(0, 0), nullptr, 0, w, W, rc, tokens, apply_case, out, ids, bits, false);
         else
             *bits = PV_ST_DECODE;
         __syncthreads();
@@ -1399,6 +1461,10 @@ __global__ void __launch_bounds__(WAVE) light_decode_kernel(pv_dev_cohort D, con
                                                           SampleIn X, HeavyList HL) {
     const uint64_t slot = (uint64_t)blockIdx.x * WAVE + threadIdx.x;
     const uint32_t lane = lane_id();
+    // A heavy wave's literal loop takes three of four vector issue slots of its SIMD, and it is the older wave: without
+    // this a light wave beside one ends only when it does, and the light lanes and the replay after them are the longer
+    // of the two.
+    __builtin_amdgcn_s_setprio(2);
     SlotHdr H{};
     bool decodable = false;
     if (slot < nslots) {
@@ -1464,7 +1530,7 @@ __global__ void __launch_bounds__(WAVE) front_kernel(pv_dev_cohort D, const int6
             const uint64_t slot = blockIdx.x;
             uint64_t w; bool rc; SlotHdr H;
             if (!entry_slot<Q>(D, wasm, wstart, nullptr, W, bpw, X, slot, w, rc, H) || rfl(H.plen) <= light_pay<Q>()) return;
-            decode_to_area<Q>(D, H, HL.area + slot * Heavy<Q>::BYTES);
+            decode_to_area<Q, true>(D, H, HL.area + slot * Heavy<Q>::BYTES);
             HL.done[slot] = (uint64_t)HL.epoch | (slot << 32);
             return;
         }
@@ -1522,7 +1588,7 @@ __global__ void __launch_bounds__(WAVE) spill_kernel(pv_dev_cohort D, const int6
 template <int Q, bool DEC, class LS>
 __device__ __forceinline__ void process_slot(LS& S, const pv_dev_cohort& D, const SlotHdr& H, uint32_t state, const uint8_t* slot_pre,
                                              uint2 op0, const uint8_t* hs, uint32_t hnops, uint64_t w, uint32_t W, bool rc, int tokens,
-                                             int apply_case, void* out, const int64_t* ids, int* status) {
+                                             int apply_case, void* out, const int64_t* ids, int* status, bool urgent) {
     constexpr bool SPAN = LS::SPAN;           // false: no staged reference span, no literal bytes in LDS (HBM / L2 reads)
     constexpr bool WINB = LS::WIN;            // blk / lower start at block position xb (a multiple of 32)
     static_assert(SPAN || !DEC, "the wave decoder needs the staged span");
@@ -1664,8 +1730,9 @@ __device__ __forceinline__ void process_slot(LS& S, const pv_dev_cohort& D, cons
     } else if constexpr (DEC) if (plen >= 3) {
         refill(d);
         d.x = (uint32_t)(d.buf & 0xFFFFFF); d.buf >>= 24; d.cnt -= 3; d.p = 3;
-        // a long payload is a long serial chain that bounds its launch: its wave issues ahead of the short-lived ones
-        if (plen > HEAVY_PAY) __builtin_amdgcn_s_setprio(3);
+        // a long payload is a long serial chain that bounds its launch (urgent: not where light lanes and a replay run
+        // beside it): its wave issues ahead of the short-lived ones
+        if (urgent && plen > HEAVY_PAY) __builtin_amdgcn_s_setprio(3);
         DecMem<Q, false> M; M.S = &S; M.blk = nullptr; M.big = (const uint16_t*)(S.aux + bmis);
         nops = (int)rfl((uint32_t)decode_block(M, OP, d, SR, gtab, R, blen, g0c, g0d));
         __builtin_amdgcn_s_setprio(0);
@@ -2175,11 +2242,11 @@ __device__ __forceinline__ void window_slot(LS& S, const pv_dev_cohort& D, const
         // byte reference to read from: there the span is staged and unpacked.
         if (state == SLOT_DONE && slot_pre && !(D.form & PV_FORM_PACKED_REF)) {
             process_slot<Q, false>(*reinterpret_cast<LdsLite<Q>*>(&S), D, H, state, slot_pre, op0, hs, hnops, w, W, rc, tokens, apply_case,
-                                   out, ids, status);
+                                   out, ids, status, false);
             return;
         }
     }
-    process_slot<Q, DEC>(S, D, H, state, slot_pre, op0, hs, hnops, w, W, rc, tokens, apply_case, out, ids, status);
+    process_slot<Q, DEC>(S, D, H, state, slot_pre, op0, hs, hnops, w, W, rc, tokens, apply_case, out, ids, status, true);
 }
 
 template <int Q, bool DEC, bool LITE = false, bool WINDOW = false>
