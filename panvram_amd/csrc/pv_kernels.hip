@@ -2401,7 +2401,7 @@ hipError_t launch(const pv_dev_cohort& D, const int64_t* wa, const int64_t* ws, 
                   const SampleIn& X, hipEvent_t ev_mid, hipEvent_t ev_end, hipStream_t st, bool may_fork) {
     bool dec = true;                                    // windows_kernel with the wave decoder
     uint32_t xshift = ~0u;
-    const Fork* fs = nullptr;                           // spill_kernel on a side stream, joined after windows_kernel
+    const Fork* fs = nullptr;                           // spill_kernel's list part and windows_kernel on side streams
     const Fork* fh = nullptr;                           // heavy_kernel on a side stream, joined after windows_kernel
     if (slotbuf && (nslots <= small_slots<Q>() || !HL.cap)) {
         // one kernel: the heavy role's waves (one per slot; none without a heavy list), then the light waves
@@ -2457,9 +2457,11 @@ hipError_t launch(const pv_dev_cohort& D, const int64_t* wa, const int64_t* ws, 
                 if (e != hipSuccess) return e;
             }
         } else {
-            // no heavy areas: a side stream does the list's long blocks whole from the start, beside the light lanes;
-            // a second one the lanes' spilled slots once the lanes are done; both beside the replay (which leaves all
-            // those slots to them) and joined after it
+            // no heavy areas: a side stream does the list's long blocks whole from the start, beside the light lanes; the
+            // lanes' spilled slots follow the lanes on the call's stream, and the replay (which leaves all those slots to
+            // the two) runs beside them on a second side stream. In that order: the whole-slot waves need 50 KB of LDS
+            // each and the replay's fill every CU, so a pass that the replay starts before waits for its end (config 3's
+            // batch: the lanes' pass 415 us beside a replay of 320 when it started 6 us after it).
             if (f) hipExtLaunchKernelGGL((spill_kernel<Q>), dim3(sw), dim3(WAVE), 0, f->side, nullptr, f->join, 0u, D, wa, ws, W, bpw, X, HL, rc,
                                          tokens, apply_case, out, ids, (int*)status, (uint32_t)SPILL_LIST);
             else hipLaunchKernelGGL((spill_kernel<Q>), dim3(sw), dim3(WAVE), 0, st, D, wa, ws, W, bpw, X, HL, rc, tokens, apply_case, out, ids,
@@ -2472,10 +2474,8 @@ hipError_t launch(const pv_dev_cohort& D, const int64_t* wa, const int64_t* ws, 
             e = hipGetLastError();
             if (e == hipSuccess && f) e = hipStreamWaitEvent(f->side2, f->lanes, 0);
             if (e != hipSuccess) return e;
-            if (f) hipExtLaunchKernelGGL((spill_kernel<Q>), dim3(sw), dim3(WAVE), 0, f->side2, nullptr, f->join2, 0u, D, wa, ws, W, bpw, X, HL, rc,
-                                         tokens, apply_case, out, ids, (int*)status, (uint32_t)SPILL_LANES);
-            else hipLaunchKernelGGL((spill_kernel<Q>), dim3(sw), dim3(WAVE), 0, st, D, wa, ws, W, bpw, X, HL, rc, tokens, apply_case, out, ids,
-                                    (int*)status, (uint32_t)SPILL_LANES);
+            hipLaunchKernelGGL((spill_kernel<Q>), dim3(sw), dim3(WAVE), 0, st, D, wa, ws, W, bpw, X, HL, rc, tokens, apply_case, out, ids,
+                               (int*)status, (uint32_t)SPILL_LANES);
             e = hipGetLastError();
             if (e != hipSuccess) return e;
             fs = f;
@@ -2496,6 +2496,10 @@ hipError_t launch(const pv_dev_cohort& D, const int64_t* wa, const int64_t* ws, 
         hipExtLaunchKernelGGL(kern, dim3((uint32_t)nslots), dim3(WAVE), dyn, st, ev_mid, ev_end, 0u, D, wa, ws, W, bpw, rc,
                               tokens, apply_case, out, ids, (int*)status, (const uint8_t*)slotbuf, (const uint64_t*)HL.done, (const uint8_t*)HL.area, xshift, HL.epoch,
                               fh ? 1u : 0u);
+    } else if (fs) {
+        hipExtLaunchKernelGGL(kern, dim3((uint32_t)nslots), dim3(WAVE), dyn, fs->side2, nullptr, fs->join2, 0u, D, wa, ws, W, bpw, rc,
+                              tokens, apply_case, out, ids, (int*)status, (const uint8_t*)slotbuf, (const uint64_t*)HL.done, (const uint8_t*)HL.area, xshift, HL.epoch,
+                              0u);
     } else {
         if (ev_mid) { const hipError_t e = hipEventRecord(ev_mid, st); if (e != hipSuccess) return e; }
         hipLaunchKernelGGL(kern, dim3((uint32_t)nslots), dim3(WAVE), dyn, st, D, wa, ws, W, bpw, rc, tokens, apply_case, out,
