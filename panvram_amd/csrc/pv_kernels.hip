@@ -758,120 +758,128 @@ __device__ __forceinline__ void heavy_mark(SlotHdr& H, uint32_t i) {
 }
 __device__ __forceinline__ uint32_t heavy_index(const SlotHdr& H) { return ((H.state >> 8) << 16) | (H.counts & 0xFFFFu); }
 
-// A light lane's rANS decoder. At Q <= 4096 the whole payload (at most LIGHT_PAY bytes) and the bytes the refills
-// read past its end are loaded into registers when the lane starts, with 16-byte loads issued together, so that no
-// refill waits on memory in the middle of the decode (a payload read is an HBM miss: the pool is read once per call).
-// At Q = 16384 (payloads of up to 64 bytes) the twenty registers that would take cost more occupancy than the refills
-// cost (config 3's batch 0.86 -> 1.08 ms with them), so the refills read the payload there (LDecMem).
-template <uint32_t NW> struct LDec {
-    uint32_t x, p, n;         // state, payload bytes consumed, payload length
-    uint64_t buf;             // the next cnt payload bytes, first in the low byte
-    uint32_t cnt;
-    bool bad;
-    uint32_t E[NW];           // the payload bytes after buf, four per word (zeros past the loaded ones)
+// A light lane's rANS decoder. The lanes of a wave are at different symbols, so a wave issues the union of their paths:
+// its time is its instructions (about 15 thousand per wave before this form) and the round trips between them. Hence:
+// no branch per symbol (a failure is kept in `bad` and looked at once per copy; what is decoded after it is bounded and
+// thrown away), one 64-bit shift of (state, next four payload bytes) per renormalisation, and no memory round trip of
+// its own for the payload: it sits in LDS (staged with 16-byte loads when the lane starts), the two words around its
+// next byte are read right after each symbol and wait there while the next symbol's table entry is on its way.
+template <int Q> struct LightLds {
+    static constexpr uint32_t LOAD = Q == 16384 ? 80 : 48;             // payload bytes staged: light_pay() and the words past it
+    static constexpr uint32_t PW = LOAD / 4 + 1, LW = 5, OW = 9;       // words per lane (odd strides: no bank twice)
+    uint32_t pay[WAVE * PW];
+    uint32_t lit[WAVE * LW];                                           // literal bytes from the 16-byte boundary at or below the count
+    uint32_t ops[WAVE * OW];                                           // ops from the multiple of four at or below the count
+    static_assert(LOAD >= light_pay<Q>() + 8, "payload staging");
 };
-// four more payload bytes from the register queue
-template <uint32_t NW> __device__ __forceinline__ void l_refill(LDec<NW>& d) {
-    d.buf |= (uint64_t)d.E[0] << (8 * d.cnt); d.cnt += 4;
-#pragma unroll
-    for (uint32_t i = 0; i + 1 < NW; i++) d.E[i] = d.E[i + 1];
-    d.E[NW - 1] = 0;
-}
-// the payload at g into the queue (reads past the payload land in the pool's padding), then the initial state: its
-// first three bytes
-template <uint32_t NW> __device__ __forceinline__ void l_start(LDec<NW>& d, const uint8_t* g, uint32_t plen) {
-#pragma unroll
-    for (uint32_t k = 0; k < NW / 4; k++) {
-        const v4u v = gload16(g + 16 * k);
-        d.E[4 * k] = v.x; d.E[4 * k + 1] = v.y; d.E[4 * k + 2] = v.z; d.E[4 * k + 3] = v.w;
-    }
-    d.n = plen; d.bad = false; d.buf = 0; d.cnt = 0;
-    l_refill(d);
-    d.x = (uint32_t)(d.buf & 0xFFFFFF); d.buf >>= 24; d.cnt -= 3; d.p = 3;
-}
-struct LDecMem {
-    uint32_t x, p, n;         // state, payload bytes consumed, payload length
-    uint64_t buf;             // the next cnt payload bytes, first in the low byte
-    uint32_t cnt;
-    bool bad;
-    const uint8_t* g;         // payload
-    uint32_t q;               // payload index of the first byte not in buf
+template <int Q> struct LDec {
+    uint32_t x, p;            // state, payload bytes consumed
+    int32_t bad;              // negative once a symbol of an all-zero context came
+    uint32_t d0, d1;          // the payload words around byte p
+    const uint32_t* pay;      // the lane's payload in LDS
 };
-__device__ __forceinline__ void l_refill(LDecMem& d) {
-    const uintptr_t A = (uintptr_t)(d.g + d.q);
-    const uint32_t* w = (const uint32_t*)(A & ~(uintptr_t)3);
-    const uint64_t v = ((((uint64_t)w[1]) << 32) | w[0]) >> (8 * (A & 3));
-    d.buf |= (v & 0xFFFFFFFFull) << (8 * d.cnt); d.cnt += 4; d.q += 4;
+// v_ffbh_u32: leading zeros (-1 for 0, which a valid state never is)
+__device__ __forceinline__ uint32_t ffbh(uint32_t v) { uint32_t r; asm("v_ffbh_u32 %0, %1" : "=v"(r) : "v"(v)); return r; }
+// the words around byte p (a payload that ran out keeps to the lane's own: p > n fails the block)
+template <int Q> __device__ __forceinline__ void l_fetch(LDec<Q>& d) {
+    const uint32_t i = min(d.p >> 2, LightLds<Q>::LOAD / 4 - 2);
+    d.d0 = d.pay[i]; d.d1 = d.pay[i + 1];
 }
-__device__ __forceinline__ void l_start(LDecMem& d, const uint8_t* g, uint32_t plen) {
-    d.g = g; d.q = 0; d.n = plen; d.bad = false; d.buf = 0; d.cnt = 0;
-    l_refill(d);
-    d.x = (uint32_t)(d.buf & 0xFFFFFF); d.buf >>= 24; d.cnt -= 3; d.p = 3;
+// the four payload bytes at p, the first in the top byte
+template <int Q> __device__ __forceinline__ uint32_t l_window(const LDec<Q>& d) { return __builtin_bswap32(__builtin_amdgcn_alignbyte(d.d1, d.d0, d.p & 3)); }
+// x below 2^16: one or two bytes of the window w bring it back (a symbol leaves at least 2^4, 16 raw bits at least 1)
+template <int Q> __device__ __forceinline__ void l_norm(LDec<Q>& d, uint32_t& w) {
+    const uint32_t sh = (ffbh(d.x) - 8) & 24;
+    const uint64_t xw = (((uint64_t)d.x << 32) | w) << sh;
+    d.x = (uint32_t)(xw >> 32); w = (uint32_t)xw;
+    d.p += sh >> 3;
 }
-template <class LD> __device__ __forceinline__ void l_renorm(LD& d) {
-    if (d.x >= pvc::RANS_L) return;
-    if (d.cnt < 2) l_refill(d);
-    if (d.p >= d.n) { d.bad = true; return; }
-    d.x = (d.x << 8) | (uint32_t)(d.buf & 0xFF); d.buf >>= 8; d.cnt--; d.p++;
-    if (d.x >= pvc::RANS_L) return;
-    if (d.p >= d.n) { d.bad = true; return; }
-    d.x = (d.x << 8) | (uint32_t)(d.buf & 0xFF); d.buf >>= 8; d.cnt--; d.p++;
-}
-// small context: cum[0..7] in one 16-byte load; the symbol is the number of cum[1..6] <= slot
-template <class LD> __device__ __forceinline__ uint32_t l_sym_small(LD& d, const uint8_t* tab, uint32_t ctx) {
-    const uint4 r = *(const uint4*)(tab + 2 * pvc::row_of((int)ctx));
-    const uint32_t slot = d.x & (pvc::M - 1);
-    const uint32_t s = (uint32_t)(slot >= (r.x >> 16)) + (uint32_t)(slot >= (r.y & 0xFFFF)) + (uint32_t)(slot >= (r.y >> 16)) +
-                       (uint32_t)(slot >= (r.z & 0xFFFF)) + (uint32_t)(slot >= (r.z >> 16)) + (uint32_t)(slot >= (r.w & 0xFFFF));
-    const uint64_t X0 = ((uint64_t)r.y << 32) | r.x, X1 = ((uint64_t)r.w << 32) | r.z;
-    const uint32_t lo = (uint32_t)((s < 4 ? X0 >> (16 * s) : X1 >> (16 * (s - 4))) & 0xFFFF);
-    const uint32_t hi = (uint32_t)((s + 1 < 4 ? X0 >> (16 * (s + 1)) : X1 >> (16 * (s - 3))) & 0xFFFF);
-    const uint32_t f = hi - lo;
-    if (!f) { d.bad = true; return s; }
+// small context: cum[0..7] in one 16-byte load. The symbol is the number of cum[1..6] <= slot: the sign bits of the four
+// half-word pairs slot - cum; its range is two neighbouring half words of the row.
+template <int Q> __device__ __forceinline__ uint32_t l_sym_small(LDec<Q>& d, const uint8_t* tab, uint32_t row) {
+    typedef uint16_t u16x2 __attribute__((ext_vector_type(2)));
+    const uint4 r = *(const uint4*)(tab + 16 * row);
+    const uint32_t slot = d.x & (pvc::M - 1), both = slot * 0x10001u;
+    auto over = [&](uint32_t c) -> uint32_t {                           // 1 per half word of c that is over slot
+        const u16x2 t = __builtin_bit_cast(u16x2, both) - __builtin_bit_cast(u16x2, c);
+        return (uint32_t)__popc(__builtin_bit_cast(uint32_t, t) & 0x80008000u);
+    };
+    const uint32_t s = 7u - over(r.x) - over(r.y) - over(r.z) - over(r.w);       // (7 in an all-zero context)
+    const uint32_t a = s < 2 ? r.x : s < 4 ? r.y : r.z, b = s < 2 ? r.y : s < 4 ? r.z : r.w;
+    const uint32_t lh = __builtin_amdgcn_alignbit(b, a, 16 * (s & 1));           // cum[s] | cum[s + 1] << 16
+    const uint32_t lo = lh & 0xFFFF, f = (lh >> 16) - lo;
+    d.bad = min(d.bad, (int32_t)(r.w >> 16) - 1);
     d.x = f * (d.x >> pvc::PROB_BITS) + slot - lo;
-    l_renorm(d);
+    uint32_t w = l_window(d);
+    l_norm(d, w);
+    l_fetch(d);
     return s;
 }
-// big context k (0..14): the slot's bucket entry gives the symbol and its range for a slot among the entry's first three
-// symbols (one load); past them, step along the row from the fourth
-template <class LD> __device__ __forceinline__ uint32_t l_sym_big(LD& d, const uint8_t* tab, uint32_t k) {
+// A value of big context k (0..14): its symbol, then the raw bits of its bucket, low 16 first. The slot's bucket entry
+// gives the symbol and its range for a slot among the entry's first three symbols (one load); past them, step along
+// the row from the fourth.
+template <int Q> __device__ __forceinline__ uint32_t l_value(LDec<Q>& d, const uint8_t* tab, uint32_t k) {
     const uint32_t slot = d.x & (pvc::M - 1);
     const uint64_t e = ((const uint64_t*)(tab + pvc::DIRECT_OFF))[k * pvc::DIRECT_NB + slot / pvc::DIRECT_W];
     const uint32_t s0 = (uint32_t)e & 127, lo0 = (uint32_t)(e >> 7) & 0xFFF;
     const uint32_t e1 = (uint32_t)(e >> 19) & 0xFFF, e2 = (uint32_t)(e >> 31) & 0xFFF, e3 = (uint32_t)(e >> 43) & 0xFFF;
-    if (s0 >= (uint32_t)pvc::BIG_ALPHA) { d.bad = true; return 0; }       // an all-zero context
-    uint32_t s, lo, f;
-    if (slot <= e3) {
-        const uint32_t i1 = slot > e1, i2 = slot > e2;
-        s = s0 + i1 + i2;
-        lo = i2 ? e2 + 1 : i1 ? e1 + 1 : lo0;
-        f = (i2 ? e3 : i1 ? e2 : e1) + 1 - lo;
-    } else {
+    d.bad = min(d.bad, pvc::BIG_ALPHA - 1 - (int32_t)s0);                // an all-zero context
+    const bool i1 = slot > e1, i2 = slot > e2;
+    uint32_t s = s0 + (i1 ? 1 : 0) + (i2 ? 1 : 0);
+    uint32_t lo = i2 ? e2 + 1 : i1 ? e1 + 1 : lo0;
+    uint32_t f = (i2 ? e3 : i1 ? e2 : e1) + 1 - lo;
+    if (slot > e3 && s0 < (uint32_t)pvc::BIG_ALPHA) {
+        // eight boundaries of the row per load (a rare symbol's bucket can hold dozens; one at a time each would be a
+        // round trip): how many are at or below the slot, the distance down to the last of them and up to the next
         const uint16_t* row = (const uint16_t*)(tab + pvc::SMALL_BYTES) + k * pvc::BIG_ROW;
-        s = s0 + 3; lo = e3 + 1;
-        uint32_t hi = row[s + 1];
-        while (hi <= slot && s < (uint32_t)pvc::BIG_ALPHA - 1) { s++; lo = hi; hi = row[s + 1]; }
-        f = hi - lo;
-        if (!f || slot < lo) { d.bad = true; return s; }
+        typedef uint16_t u16x2 __attribute__((ext_vector_type(2)));
+        const u16x2 at = __builtin_bit_cast(u16x2, slot * 0x10001u), one = {1, 1};
+        u16x2 down = __builtin_bit_cast(u16x2, (slot - e3 - 1) * 0x10001u), up;
+        uint32_t n;
+        s = s0 + 3;
+        do {
+            u16x2 c[4];
+            __builtin_memcpy(c, row + min(s + 1, (uint32_t)pvc::BIG_ROW - 8u), 16);
+            uint32_t over = 0;
+            up = u16x2{0xFFFF, 0xFFFF};
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                const u16x2 t = at - c[i];
+                over += (uint32_t)__popc(__builtin_bit_cast(uint32_t, t) & 0x80008000u);
+                down = __builtin_elementwise_min(down, t);             // (a boundary over the slot: a large number)
+                up = __builtin_elementwise_min(up, (u16x2)(c[i] - at - one));
+            }
+            n = 8 - over;
+            s += n;
+        } while (n == 8 && s < (uint32_t)pvc::BIG_ALPHA);
+        lo = slot - min((uint32_t)down.x, (uint32_t)down.y);
+        f = slot + 1 + min((uint32_t)up.x, (uint32_t)up.y) - lo;
     }
     d.x = f * (d.x >> pvc::PROB_BITS) + slot - lo;
-    l_renorm(d);
-    return s;
-}
-template <class LD> __device__ __forceinline__ uint64_t l_draw(LD& d, uint32_t nb) {
-    uint64_t v = 0; uint32_t sh = 0;
-    while (nb && !d.bad) {
-        const uint32_t k = nb > 16 ? 16 : nb;
-        const uint32_t b = d.x & ((1u << k) - 1); d.x >>= k;
-        l_renorm(d);
-        v |= (uint64_t)b << sh; sh += k; nb -= k;
+    uint32_t w = l_window(d);
+    l_norm(d, w);
+    const uint32_t t = s - 16, nb = s < 16 ? 0u : (t >> 2) + 2, n0 = min(nb, 16u);
+    uint32_t v = __builtin_amdgcn_ubfe(d.x, 0, n0);
+    d.x >>= n0;
+    l_norm(d, w);
+    l_fetch(d);
+    if (nb > 16) {
+        w = l_window(d);
+        v |= __builtin_amdgcn_ubfe(d.x, 0, nb - 16) << 16;
+        d.x >>= nb - 16;
+        l_norm(d, w);
+        l_fetch(d);
     }
-    return v;
+    return s < 16 ? s : ((4u | (t & 3)) << (nb & 31)) | v;
 }
-template <class LD> __device__ __forceinline__ uint64_t l_dval(LD& d, const uint8_t* tab, uint32_t k) {
-    const uint32_t s = l_sym_big(d, tab, k);
-    if (d.bad) return 0;
-    return pvc::unbucket(s, l_draw(d, pvc::nbits_of(s)));
+// n (8 or 16) raw bits, twice for the 32-bit positions
+template <int Q> __device__ __forceinline__ uint32_t l_raw(LDec<Q>& d, uint32_t n) {
+    uint32_t w = l_window(d);
+    const uint32_t v = __builtin_amdgcn_ubfe(d.x, 0, n);
+    d.x >>= n;
+    l_norm(d, w);
+    l_fetch(d);
+    return v;
 }
 // the block table entry of block b of archive record ar (plain or compact form), one lane at a time
 __device__ __forceinline__ void l_block(const pv_dev_cohort& D, const int64_t* ar, uint64_t b, uint64_t bb, uint32_t& poff, uint32_t& plen,
@@ -1273,178 +1281,155 @@ __global__ void __launch_bounds__(WAVE) slot_kernel(pv_dev_cohort D, const int64
     }
 }
 
-// A short payload's decode by the slot's lane (H: the slot's header, state SLOT_WAVE, payload of 3 to LIGHT_PAY
+// A short payload's decode by the slot's lane (H: the slot's header, state SLOT_WAVE, payload of 3 to light_pay()
 // bytes): the block's ops and literal bytes to the slot's record, state SLOT_DONE with the counts, or SLOT_FAILED.
-// True when the block needs more ops or literals than a record holds (the header is then unchanged).
-// LT: the assembly's model table is in LDS at `ltab` (a one-window call's, staged by its wave), else read from HBM.
+// True when the block needs more ops or literals than a record holds, or starts from a state below 2^16 (the header
+// is then unchanged). LT: the assembly's model table is in LDS at `ltab` (its wave staged it), else read from HBM.
 template <int Q, bool LT = false>
-__device__ __forceinline__ bool light_lane(const pv_dev_cohort& D, uint64_t slot, uint8_t* slotbuf, SlotHdr& H, const uint8_t* ltab = nullptr) {
-    bool spilled = false;
-    do {
-        const uint32_t blen = H.counts >> 16, plen = H.plen;
-        const int64_t a = H.a, stv = H.stv;
-        const uint8_t* tab = LT ? ltab : D.tab + (uint64_t)a * pvc::GTAB_BYTES;
-        RefView R; R.g = D.ref; R.n = D.ref_n; R.wbase = 0; R.wlen = 0;
-        R.pw = (D.form & PV_FORM_PACKED_REF) ? D.pw : nullptr; R.pes = D.pes; R.pel = D.pel; R.peb = D.peb; R.peix = D.peix; R.pne = D.pne;
-        // at Q <= 4096 the payload and the (at most five) bytes the refills read past its end, in 16-byte loads
-        typename std::conditional<Q == 16384, LDecMem, LDec<4 * ((LIGHT_PAY + 5 + 15) / 16)>>::type d;
-        l_start(d, D.P + H.payoff, plen);
-        uint2* ops = (uint2*)(slotbuf + slot * SLOT_BYTES + SL_OPS);
-        uint8_t* lits = slotbuf + slot * SLOT_BYTES + SL_LIT;
-        // the four-entry move-to-front diagonal cache (csrc/refrel3.h:94-102), one lane's own
-        int64_t cc0 = stv >> 1, cc1 = 0, cc2 = 0, cc3 = 0; uint32_t cd0 = (uint32_t)(stv & 1), cd1 = 0, cd2 = 0, cd3 = 0; int cn = 1;
-        int prevk = -1; uint32_t o = 0, nops = 0, nlit = 0;
-        bool spill = false;
-        // The record is written in 32-byte groups of four ops and 16-byte groups of literal bytes (the partial ones at
-        // the end): a store counts in the wave's vector memory counter until it completes, so each store ahead of a
-        // table read would hold back the wait for that read.
-        uint2 opb0 = make_uint2(0, 0), opb1 = opb0, opb2 = opb0;      // ops nops & ~3 .. nops - 1 (not yet stored)
-        uint64_t lacc0 = 0, lacc1 = 0;                                // literal bytes from the 16-byte boundary at or below nlit
-        auto put_op = [&](uint2 v) {
-            switch (nops & 3) {
-                case 0: opb0 = v; break;
-                case 1: opb1 = v; break;
-                case 2: opb2 = v; break;
-                default:
-                    *(uint4*)(ops + (nops - 3)) = make_uint4(opb0.x, opb0.y, opb1.x, opb1.y);
-                    *(uint4*)(ops + (nops - 1)) = make_uint4(opb2.x, opb2.y, v.x, v.y);
+__device__ __forceinline__ bool light_lane(const pv_dev_cohort& D, uint64_t slot, uint8_t* slotbuf, SlotHdr& H, LightLds<Q>& S, const uint8_t* ltab = nullptr) {
+    using LL = LightLds<Q>;
+    const uint32_t l = lane_id(), blen = H.counts >> 16, plen = H.plen;
+    const uint8_t* tab = LT ? ltab : D.tab + (uint64_t)H.a * pvc::GTAB_BYTES;
+    const bool packed = D.form & PV_FORM_PACKED_REF;
+    RefView R; R.g = D.ref; R.n = D.ref_n; R.wbase = 0; R.wlen = 0;
+    R.pw = packed ? D.pw : nullptr; R.pes = D.pes; R.pel = D.pel; R.peb = D.peb; R.peix = D.peix; R.pne = D.pne;
+    LDec<Q> d;
+    uint32_t* pay = S.pay + l * LL::PW;
+    {
+        const uint8_t* g = D.P + H.payoff;                             // (reads past the payload land in the pool's padding)
+        v4u v[LL::LOAD / 16];
+#pragma unroll
+        for (uint32_t k = 0; k < LL::LOAD / 16; k++) v[k] = gload16(g + 16 * k);
+#pragma unroll
+        for (uint32_t k = 0; k < LL::LOAD / 16; k++) { pay[4 * k] = v[k].x; pay[4 * k + 1] = v[k].y; pay[4 * k + 2] = v[k].z; pay[4 * k + 3] = v[k].w; }
+        d.x = v[0].x & 0xFFFFFF; d.p = 3; d.bad = 0; d.pay = pay;
+        d.d0 = v[0].x; d.d1 = v[0].y;
+    }
+    if (d.x < pvc::RANS_L) return true;                                // (a corrupt payload) one byte at a time, by the wave decoder
+    uint2* ops = (uint2*)(slotbuf + slot * SLOT_BYTES + SL_OPS);
+    uint8_t* lits = slotbuf + slot * SLOT_BYTES + SL_LIT;
+    uint32_t* lop = S.ops + l * LL::OW;
+    uint32_t* lit = S.lit + l * LL::LW;
+    // The record is written in 32-byte groups of four ops and 16-byte groups of literal bytes, gathered in LDS (the
+    // partial ones at the end): a store counts in the wave's vector memory counter until it completes, so each store
+    // ahead of a table read would hold back the wait for that read.
+    uint32_t o = 0, nops = 0, nlit = 0;
+    auto put_op = [&](uint32_t src, uint32_t w1) {
+        lop[2 * (nops & 3)] = src; lop[2 * (nops & 3) + 1] = w1;
+        if ((nops & 3) == 3) {
+            *(uint4*)(ops + (nops - 3)) = make_uint4(lop[0], lop[1], lop[2], lop[3]);
+            *(uint4*)(ops + (nops - 1)) = make_uint4(lop[4], lop[5], lop[6], lop[7]);
+        }
+        nops++;
+    };
+    // the four-entry move-to-front diagonal cache (csrc/refrel3.h:94-102), one lane's own: c << 1 | strand
+    int64_t e0 = H.stv, e1 = 0, e2 = 0, e3 = 0;
+    uint32_t cn = 1, kc = 0;                                           // entries held; kclass of the copy before
+    bool ok = true, spill = false;
+    while (o < blen) {
+        const uint32_t ll = l_value(d, tab, kc);
+        if (ll > blen - o) { ok = false; break; }
+        if (ll) {
+            if (nops >= LOPS || nlit + ll > LLIT) { spill = true; break; }
+            put_op(nlit, o | (ll << 15));
+            // a short run's contexts are the reference bases its diagonal predicts, at most 8 consecutive positions: one
+            // 8-byte load, its bytes turned into the run's order, where all of them lie in the (byte) reference
+            const bool shrt = ll <= 8;
+            const uint32_t dir = (uint32_t)e0 & 1;
+            const int64_t q0 = pvc::diag_locus(e0 >> 1, dir, o), qb = dir ? q0 - (int64_t)ll + 1 : q0;
+            const bool fast = shrt && !packed && qb >= 0 && (uint64_t)qb + ll <= R.n;
+            uint64_t pre = 0;
+            if (fast) {
+                __builtin_memcpy(&pre, R.g + qb, 8);
+                if (dir) pre = __builtin_bswap64(pre) >> (8 * (8 - ll));
             }
-            nops++;
-        };
-        constexpr uint32_t ACGTN = 'A' | ('C' << 8) | ('G' << 16) | ('T' << 24);
-        while (o < blen && !d.bad && !spill) {
-            const uint64_t ll = l_dval(d, tab, (uint32_t)pvc::kclass(prevk));
-            if (d.bad || ll > blen - o) { d.bad = true; break; }
-            if (ll) {
-                if (nops >= LOPS || nlit + ll > LLIT) { spill = true; break; }
-                put_op(make_uint2(nlit, o | ((uint32_t)ll << 15)));
-                // a short run's contexts read the reference bases its diagonal predicts, at most 8 consecutive positions:
-                // the 16 bytes from the 8-byte boundary below the lowest one, loaded once (the device reference carries
-                // 1 KiB of padding), instead of one dependent load per literal
-                uint64_t pre0 = 0, pre1 = 0; int64_t pbase = -1;
-                if (ll <= 8 && !R.pw) {
-                    const int64_t q0 = pvc::diag_locus(cc0, cd0, o), qb = cd0 ? q0 - (int64_t)ll + 1 : q0;
-                    if (qb >= 0 && (uint64_t)qb < R.n) {
-                        pbase = qb & ~(int64_t)7;
-                        const uint64_t* pp = (const uint64_t*)(R.g + pbase);
-                        pre0 = pp[0]; pre1 = pp[1];
+            uint32_t r = 16;
+            for (uint32_t k = 0; k < ll; k++) {
+                uint32_t row = SR_LIT2 + r;
+                if (shrt) {
+                    uint32_t byte = (uint32_t)pre & 0xFF;
+                    pre >>= 8;
+                    if (!fast) {
+                        const int64_t q = pvc::diag_locus(e0 >> 1, dir, o + k);
+                        byte = q >= 0 && (uint64_t)q < R.n ? (packed ? packed_at(R, (uint64_t)q) : R.g[q]) : 0;
                     }
+                    // the base code: bits 1-2 of A C G T are 0 1 3 2; any other byte is 4
+                    uint32_t c = (byte >> 1) & 3;
+                    c ^= c >> 1;
+                    const uint32_t rb = ((ACGT >> (8 * c)) & 0xFF) == byte ? (dir ? 3 - c : c) : 4;
+                    row = SR_LITR + rb * 2 + (k == 0 ? 1 : 0);
                 }
-                uint32_t r = 16;
-                for (uint32_t k = 0; k < (uint32_t)ll && !d.bad; k++) {
-                    uint32_t ctx;
-                    if (ll <= 8) {
-                        const int64_t q = pvc::diag_locus(cc0, cd0, o + k);
-                        uint32_t rb = 4;
-                        if (q >= 0 && (uint64_t)q < R.n) {
-                            uint32_t byte;
-                            if (pbase >= 0) {
-                                const uint32_t t = (uint32_t)(q - pbase);          // 0..15: the run lies in the 16 bytes
-                                byte = (uint32_t)((t < 8 ? pre0 >> (8 * t) : pre1 >> (8 * (t - 8))) & 0xFF);
-                            } else {
-                                byte = R.pw ? packed_at(R, (uint64_t)q) : R.g[q];
-                            }
-                            rb = base_code(byte, cd0);
-                        }
-                        ctx = pvc::C_LITR + rb * 2 + (k == 0 ? 1 : 0);
-                    } else {
-                        ctx = pvc::C_LIT2 + r;
-                    }
-                    const uint32_t sy = l_sym_small(d, tab, ctx);
-                    if (d.bad) break;
-                    uint32_t byte = sy < 4 ? (ACGTN >> (8 * sy)) & 0xFF : 'N';
-                    if (sy == 5) byte = (uint32_t)l_draw(d, 8);
-                    const uint32_t q16 = nlit + k;
-                    if (q16 & 8) lacc1 |= (uint64_t)(byte & 0xFF) << (8 * (q16 & 7));
-                    else lacc0 |= (uint64_t)(byte & 0xFF) << (8 * (q16 & 7));
-                    if ((q16 & 15) == 15) {
-                        *(uint4*)(lits + (q16 & ~15u)) = make_uint4((uint32_t)lacc0, (uint32_t)(lacc0 >> 32), (uint32_t)lacc1, (uint32_t)(lacc1 >> 32));
-                        lacc0 = lacc1 = 0;
-                    }
-                    r = ((r * 4) + (sy < 4 ? sy : 0)) & 15;
-                }
-                if (d.bad) break;
-                nlit += (uint32_t)ll; o += (uint32_t)ll;
+                const uint32_t sy = l_sym_small(d, tab, row);
+                uint32_t byte = sy < 4 ? (ACGT >> (8 * sy)) & 0xFF : 'N';
+                if (sy == 5) byte = l_raw(d, 8);
+                ((uint8_t*)lit)[nlit & 15] = (uint8_t)byte;
+                if ((nlit & 15) == 15) *(uint4*)(lits + (nlit & ~15u)) = make_uint4(lit[0], lit[1], lit[2], lit[3]);
+                nlit++;
+                r = ((r * 4) + (sy < 4 ? sy : 0)) & 15;
             }
+            o += ll;
             if (o == blen) break;
-            const int kind = (int)l_sym_small(d, tab, pvc::C_KIND + pvc::llc(ll) * 4 + pvc::kclass(prevk));
-            if (d.bad || kind > pvc::K_FLIP) { d.bad = true; break; }
-            // One decode path for every kind, since the lanes of a wave hold different kinds and a branch per kind would
-            // run each kind's decode in turn: the kind's small symbol (REP, FLIP: the cache entry; ABS: the strand), then
-            // its value (DELTA, REP, FLIP: the diagonal shift, zigzag coded; SELF: the distance; ABS: 32 raw bits), in
-            // the order they were coded (csrc/refrel3.h:136-142)
-            uint32_t aux = 0;
-            if (kind == pvc::K_REP || kind == pvc::K_FLIP || kind == pvc::K_ABS)
-                aux = l_sym_small(d, tab, kind == pvc::K_REP ? pvc::C_REPK : kind == pvc::K_FLIP ? pvc::C_FLIPK : pvc::C_DIR);
-            uint64_t val = 0;
-            if (!d.bad && kind == pvc::K_ABS) {
-                val = l_draw(d, 32);
-            } else if (!d.bad && kind != pvc::K_CONT) {
-                val = l_dval(d, tab, kind == pvc::K_DELTA ? 4 + (ll == 0 ? 0 : 1) : kind == pvc::K_REP ? 6 : kind == pvc::K_SELF ? 7 : 14);
-            }
-            if (d.bad) break;
-            uint64_t p = 0; uint32_t dir = 0; int ki = 0; int64_t dd = 0; uint64_t dist = 0;
-            if (kind == pvc::K_ABS) {
-                dir = aux; p = val;
-            } else if (kind == pvc::K_SELF) {
-                dist = val;
-            } else if (kind != pvc::K_CONT) {
-                dd = pvc::unzigzag(val);
-                ki = kind == pvc::K_REP ? 1 + (int)aux : kind == pvc::K_FLIP ? (int)aux : 0;
-                if (ki >= cn) { d.bad = true; break; }
-            }
-            const uint64_t L = l_dval(d, tab, 8 + (uint32_t)kind) + pvc::MIN_LEN;
-            if (d.bad || L > blen - o) { d.bad = true; break; }
-            uint32_t okind; uint64_t osrc;
-            if (kind == pvc::K_SELF) {
-                if (dist == 0 || dist > o) { d.bad = true; break; }
-                okind = 2; osrc = o - dist;
-            } else {
-                const int k = kind == pvc::K_REP ? ki : kind == pvc::K_FLIP ? ki : 0;
-                const int64_t gc = k == 0 ? cc0 : k == 1 ? cc1 : k == 2 ? cc2 : cc3;
-                const uint32_t gd = k == 0 ? cd0 : k == 1 ? cd1 : k == 2 ? cd2 : cd3;
-                if (kind == pvc::K_FLIP) {
-                    dir = gd ^ 1;
-                    const int64_t e = pvc::diag_locus(gc, gd, o) + dd; if (e < 0) { d.bad = true; break; } p = (uint64_t)e;
-                } else if (kind != pvc::K_ABS) {
-                    dir = gd;
-                    const int64_t e = pvc::diag_expect(gc, gd, o, L) + dd; if (e < 0) { d.bad = true; break; } p = (uint64_t)e;
-                }
-                if (p > R.n || L > R.n - p) { d.bad = true; break; }
-                okind = dir ? 3 : 1; osrc = p;
-                // move-to-front push of the copy's diagonal
-                const int64_t nc = pvc::diag_of(dir, p, o, L);
-                int jx = cn;
-                if (cn > 0 && cc0 == nc && cd0 == dir) jx = 0;
-                else if (cn > 1 && cc1 == nc && cd1 == dir) jx = 1;
-                else if (cn > 2 && cc2 == nc && cd2 == dir) jx = 2;
-                else if (cn > 3 && cc3 == nc && cd3 == dir) jx = 3;
-                if (jx == cn) { if (cn < 4) cn++; jx = cn - 1; }
-                if (jx >= 3) { cc3 = cc2; cd3 = cd2; }
-                if (jx >= 2) { cc2 = cc1; cd2 = cd1; }
-                if (jx >= 1) { cc1 = cc0; cd1 = cd0; }
-                cc0 = nc; cd0 = dir;
-            }
-            // (at Q = 16384 a self copy goes to the whole-slot pass too: the replay there keeps only the window's part)
-            if (nops >= LOPS || (okind == 2 && D.Q == 16384)) { spill = true; break; }
-            put_op(make_uint2((uint32_t)osrc, o | ((uint32_t)L << 15) | (okind << 30)));
-            o += (uint32_t)L; prevk = kind;
         }
-        if (spill) { spilled = true; break; }                   // more ops or literals than a slot record holds
-        if (d.bad || d.x != pvc::RANS_L || d.p != d.n) { H.state = SLOT_FAILED; break; }
-        if (nops & 3) {
-            const uint32_t b = nops & ~3u;
-            ops[b] = opb0;
-            if ((nops & 3) > 1) ops[b + 1] = opb1;
-            if ((nops & 3) > 2) ops[b + 2] = opb2;
+        const uint32_t kind = l_sym_small(d, tab, SR_KIND + (uint32_t)pvc::llc(ll) * 4 + kc);
+        if (kind > (uint32_t)pvc::K_FLIP) { ok = false; break; }
+        // One decode path for every kind, since the lanes of a wave hold different kinds and a branch per kind would
+        // run each kind's decode in turn: the kind's small symbol (REP, FLIP: the cache entry; ABS: the strand), then
+        // its value (DELTA, REP, FLIP: the diagonal shift, zigzag coded; SELF: the distance; ABS: 32 raw bits), in
+        // the order they were coded (csrc/refrel3.h:136-142)
+        uint32_t aux = 0, val = 0;
+        if (kind == pvc::K_REP || kind == pvc::K_FLIP || kind == pvc::K_ABS) {
+            aux = l_sym_small(d, tab, kind == pvc::K_REP ? SR_REPK : kind == pvc::K_FLIP ? SR_FLIPK : SR_DIR);
+            if (kind == pvc::K_ABS) { val = l_raw(d, 16); val |= l_raw(d, 16) << 16; }
         }
-        if (nlit & 15)
-            *(uint4*)(lits + (nlit & ~15u)) = make_uint4((uint32_t)lacc0, (uint32_t)(lacc0 >> 32), (uint32_t)lacc1, (uint32_t)(lacc1 >> 32));
-        H.counts |= nops | nlit << 8;
-        H.state = SLOT_DONE;
-    } while (false);
-    return spilled;
+        if (kind != pvc::K_CONT && kind != pvc::K_ABS)
+            val = l_value(d, tab, kind == pvc::K_DELTA ? BR_DELTA + (ll ? 1u : 0u) : kind == pvc::K_REP ? BR_REPD : kind == pvc::K_SELF ? BR_SELF : BR_FLIPD);
+        const uint32_t L = l_value(d, tab, BR_LEN + kind) + pvc::MIN_LEN;
+        if (d.bad < 0 || d.p > plen || L > blen - o) { ok = false; break; }
+        uint32_t okind, osrc;
+        if (kind == pvc::K_SELF) {
+            if (val == 0 || val > o) { ok = false; break; }
+            okind = 2; osrc = o - val;
+        } else {
+            const uint32_t ki = kind == pvc::K_REP ? 1 + aux : kind == pvc::K_FLIP ? aux : 0;
+            if (ki >= cn) { ok = false; break; }
+            const int64_t ge = ki == 0 ? e0 : ki == 1 ? e1 : ki == 2 ? e2 : e3, gc = ge >> 1;
+            const uint32_t gd = (uint32_t)ge & 1;
+            // where the cached diagonal leads: its locus at o for a flip, else the copy's expected start
+            int64_t p = (gd ? gc - (int64_t)o : gc + (int64_t)o) + pvc::unzigzag(val);
+            if (gd && kind != pvc::K_FLIP) p -= (int64_t)L - 1;
+            uint32_t dir = kind == pvc::K_FLIP ? gd ^ 1 : gd;
+            if (kind == pvc::K_ABS) { p = (int64_t)(uint64_t)val; dir = aux; }
+            if (p < 0 || (uint64_t)p > R.n || L > R.n - (uint64_t)p) { ok = false; break; }
+            okind = dir ? 3 : 1; osrc = (uint32_t)p;
+            // move-to-front push of the copy's diagonal
+            const int64_t ne = (int64_t)((uint64_t)pvc::diag_of(dir, (uint64_t)p, o, L) << 1 | dir);
+            if (ne != e0) {
+                uint32_t j = cn > 1 && e1 == ne ? 1 : cn > 2 && e2 == ne ? 2 : cn > 3 && e3 == ne ? 3 : 4;
+                if (j == 4) { if (cn < 4) cn++; j = cn - 1; }
+                if (j >= 3) e3 = e2;
+                if (j >= 2) e2 = e1;
+                e1 = e0; e0 = ne;
+            }
+        }
+        // (at Q = 16384 a self copy goes to the whole-slot pass too: the replay there keeps only the window's part)
+        if (nops >= LOPS || (okind == 2 && Q == 16384)) { spill = true; break; }
+        put_op(osrc, o | (L << 15) | (okind << 30));
+        o += L; kc = (0xBE9u >> (2 * kind)) & 3;                       // kclass of CONT .. FLIP: 1 2 2 3 3 2
+    }
+    if (spill) return true;                                            // more ops or literals than a slot record holds
+    if (!ok || d.bad < 0 || d.x != pvc::RANS_L || d.p != plen) { H.state = SLOT_FAILED; return false; }
+    if (nops & 3) {
+        const uint32_t b = nops & ~3u;
+        ops[b] = make_uint2(lop[0], lop[1]);
+        if ((nops & 3) > 1) ops[b + 1] = make_uint2(lop[2], lop[3]);
+        if ((nops & 3) > 2) ops[b + 2] = make_uint2(lop[4], lop[5]);
+    }
+    if (nlit & 15) *(uint4*)(lits + (nlit & ~15u)) = make_uint4(lit[0], lit[1], lit[2], lit[3]);
+    H.counts |= nops | nlit << 8;
+    H.state = SLOT_DONE;
+    return false;
 }
+static_assert(pvc::kclass(0) == 1 && pvc::kclass(1) == 2 && pvc::kclass(2) == 2 && pvc::kclass(3) == 3 && pvc::kclass(4) == 3 && pvc::kclass(5) == 2, "kind classes");
 
 // The heavy waves of a large call (heavy_decode), in a kernel of their own: the light lanes then run without the
 // wave decoder's registers.
@@ -1455,7 +1440,12 @@ __global__ void __launch_bounds__(WAVE) heavy_kernel(pv_dev_cohort D, const int6
 }
 
 // The decode of the slots slot_kernel left to the light path (SLOT_WAVE with a short payload), one lane per slot.
-template <int Q>
+// LONG: a call of windows of LONG_BPW slots or more (a chromosome, a stream decode), where most waves hold slots of one
+// window and so of one assembly: such a wave stages that model table in LDS first, so that its lanes' table reads wait
+// on LDS instead of L2 (a wave of mixed assemblies reads them from HBM). Its 10 KB per wave would cost the other calls
+// half their waves per CU, and at 16 K block size hold back the whole-slot pass beside this kernel (50 KB per wave).
+constexpr uint32_t LONG_BPW = 256;
+template <int Q, bool LONG>
 __global__ void __launch_bounds__(WAVE) light_decode_kernel(pv_dev_cohort D, const int64_t* __restrict__ wasm, const int64_t* __restrict__ wstart,
                                                           uint32_t W, uint32_t bpw, uint64_t nslots, uint8_t* __restrict__ slotbuf,
                                                           SampleIn X, HeavyList HL) {
@@ -1473,24 +1463,20 @@ __global__ void __launch_bounds__(WAVE) light_decode_kernel(pv_dev_cohort D, con
         hs[0] = hp[0]; hs[1] = hp[1]; hs[2] = hp[2]; hs[3] = hp[3];
         decodable = H.state == SLOT_WAVE && H.plen <= light_pay<Q>();
     }
-    // Below 16 K block size, a wave whose slots are all of one assembly (a long window's, a stream decode's) stages that
-    // model table in LDS first, so that its lanes' table reads wait on LDS instead of L2; a wave of mixed assemblies
-    // reads them from HBM. (At 16 K the whole-slot pass runs beside this kernel and needs 50 KB of LDS per wave: the
-    // table's 10 KB per wave here would hold it back.)
-    bool spilled = false;
-    bool staged = false;
-    if constexpr (Q != 16384) {
+    __shared__ LightLds<Q> S;
+    bool spilled = false, staged = false;
+    if constexpr (LONG) {
         const uint64_t dm = __ballot(decodable);
         const uint32_t a0 = dm ? rdl(H.a, (uint32_t)__builtin_ctzll(dm)) : 0u;
         if (dm && !__ballot(decodable && H.a != a0)) {
             __shared__ __align__(16) uint8_t tl[pvc::GTAB_BYTES + 16];
             const uint32_t mis = stage(tl, D.tab + (uint64_t)a0 * pvc::GTAB_BYTES, pvc::GTAB_BYTES, pvc::GTAB_BYTES + 16);
             stage_wait();
-            if (decodable) spilled = light_lane<Q, true>(D, slot, slotbuf, H, tl + mis);
+            if (decodable) spilled = light_lane<Q, true>(D, slot, slotbuf, H, S, tl + mis);
             staged = true;
         }
     }
-    if (!staged && decodable) spilled = light_lane<Q>(D, slot, slotbuf, H);
+    if (!staged && decodable) spilled = light_lane<Q>(D, slot, slotbuf, H, S);
     // a spilled slot takes an entry after slot_kernel's long ones (one atomic per wave)
     const uint64_t m = __ballot(spilled);
     if (m && HL.cap) {
@@ -1541,6 +1527,7 @@ __global__ void __launch_bounds__(WAVE) front_kernel(pv_dev_cohort D, const int6
     SlotHdr H;
     const bool heavy = slot_header<Q>(D, wasm, wstart, W, bpw, nslots, X, slot, H);
     if (heavy) { if (HL.nworkers) heavy_mark(H, (uint32_t)slot); }
+    __shared__ LightLds<Q> S;
     if constexpr (ONE) {
         __shared__ __align__(16) uint8_t tl[pvc::GTAB_BYTES + 16];
         const uint64_t m = __ballot(!heavy && H.state == SLOT_WAVE);
@@ -1548,10 +1535,10 @@ __global__ void __launch_bounds__(WAVE) front_kernel(pv_dev_cohort D, const int6
             const uint32_t a = rdl(H.a, (uint32_t)__builtin_ctzll(m));
             const uint32_t mis = stage(tl, D.tab + (uint64_t)a * pvc::GTAB_BYTES, pvc::GTAB_BYTES, pvc::GTAB_BYTES + 16);
             stage_wait();
-            if (!heavy && H.state == SLOT_WAVE) (void)light_lane<Q, true>(D, slot, slotbuf, H, tl + mis);
+            if (!heavy && H.state == SLOT_WAVE) (void)light_lane<Q, true>(D, slot, slotbuf, H, S, tl + mis);
         }
     } else {
-        if (!heavy && H.state == SLOT_WAVE) (void)light_lane<Q>(D, slot, slotbuf, H);
+        if (!heavy && H.state == SLOT_WAVE) (void)light_lane<Q>(D, slot, slotbuf, H, S);
     }
     if (slot < nslots) {
         uint4* hv = (uint4*)(slotbuf + slot * SLOT_BYTES);
@@ -2443,7 +2430,8 @@ hipError_t launch(const pv_dev_cohort& D, const int64_t* wa, const int64_t* ws, 
             }
             e = hipGetLastError();
             if (e != hipSuccess) return e;
-            hipLaunchKernelGGL((light_decode_kernel<Q>), dim3(HL.nlight), dim3(WAVE), 0, st, D, wa, ws, W, bpw, nslots, slotbuf, X, HL);
+            auto lk = bpw >= LONG_BPW ? light_decode_kernel<Q, true> : light_decode_kernel<Q, false>;
+            hipLaunchKernelGGL(lk, dim3(HL.nlight), dim3(WAVE), 0, st, D, wa, ws, W, bpw, nslots, slotbuf, X, HL);
             e = hipGetLastError();
             if (e != hipSuccess) return e;
             if (f && !ev_mid) {
@@ -2468,9 +2456,9 @@ hipError_t launch(const pv_dev_cohort& D, const int64_t* wa, const int64_t* ws, 
                                     (int*)status, (uint32_t)SPILL_LIST);
             e = hipGetLastError();
             if (e != hipSuccess) return e;
-            if (f) hipExtLaunchKernelGGL((light_decode_kernel<Q>), dim3(HL.nlight), dim3(WAVE), 0, st, nullptr, f->lanes, 0u, D, wa, ws, W, bpw,
+            if (f) hipExtLaunchKernelGGL((light_decode_kernel<Q, false>), dim3(HL.nlight), dim3(WAVE), 0, st, nullptr, f->lanes, 0u, D, wa, ws, W, bpw,
                                          nslots, slotbuf, X, HL);
-            else hipLaunchKernelGGL((light_decode_kernel<Q>), dim3(HL.nlight), dim3(WAVE), 0, st, D, wa, ws, W, bpw, nslots, slotbuf, X, HL);
+            else hipLaunchKernelGGL((light_decode_kernel<Q, false>), dim3(HL.nlight), dim3(WAVE), 0, st, D, wa, ws, W, bpw, nslots, slotbuf, X, HL);
             e = hipGetLastError();
             if (e == hipSuccess && f) e = hipStreamWaitEvent(f->side2, f->lanes, 0);
             if (e != hipSuccess) return e;
