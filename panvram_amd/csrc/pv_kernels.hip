@@ -2805,15 +2805,20 @@ constexpr double LANE_SPIN_S = 60.0;
 // The caller's wait for a lane's mark (one lane of one wave): poll the lane's counter (system scope: signal memory
 // that another queue's packet writes) until it reaches `target`, then store the caller's mark `mark`. Bounded at
 // LANE_SPIN_S of the GPU's 100 MHz clock: past it the wave stores the mark anyway and sets status bit 4 in the call's
-// status word, so that the call reports the wait instead of returning rows that may not be complete.
+// status word, so that the call reports the wait instead of returning rows that may not be complete. The polls are
+// relaxed, with one acquire after the last, and 2,048 clocks apart: a read of signal memory takes microseconds, and the
+// CU's other waves' reads return in order behind it. At 128 clocks apart the one light wave that shared the poll's CU
+// took 125-135 us where the longest of the others took 60, and the kernel's time was that wave's (sample of 65,536
+// windows 376 us a call at 128 clocks, 360 at 1,024, 354 at 3,072; of 1,024 156, 149, 150).
 constexpr uint64_t WAIT_TICKS = (uint64_t)(LANE_SPIN_S * 100e6);
 __global__ void __launch_bounds__(WAVE) caller_wait_kernel(const uint64_t* lane, uint64_t target, uint64_t* mark, uint64_t m, int* status) {
     if (threadIdx.x != 0) return;
     const uint64_t t0 = wall_clock64();
-    while (__hip_atomic_load(lane, __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_SYSTEM) < target) {
+    while (__hip_atomic_load(lane, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM) < target) {
         if (wall_clock64() - t0 > WAIT_TICKS) { atomicOr(status, PV_ST_WAIT); break; }
-        __builtin_amdgcn_s_sleep(2);
+        __builtin_amdgcn_s_sleep(32);
     }
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "");
     __hip_atomic_store(mark, m, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 struct Sig {                                              // a lane's or a caller's progress marks
