@@ -2330,6 +2330,77 @@ __global__ void __launch_bounds__(256) sample_coords_kernel(const int64_t* __res
     }
 }
 
+// A tool that serialises kernel dispatches (rocprofv3 counter collection or thread trace, which set these variables for
+// the process they profile): a caller wait carried out as a polling kernel would then wait for a lane kernel that
+// cannot start until the poll ends, so the counter wait falls back to events there.
+bool serialised_dispatch() {
+    static const bool on = [] {
+        for (const char* v : {"ROCPROF_COUNTER_COLLECTION", "ROCPROF_COUNTERS", "ROCPROF_COUNTER_GROUPS", "ROCPROF_ADVANCED_THREAD_TRACE"}) {
+            const char* s = getenv(v);
+            if (s && *s && strcmp(s, "0") != 0 && strcasecmp(s, "false") != 0) return true;
+        }
+        return false;
+    }();
+    return on;
+}
+// One lane waits until the GPU's real-time clock (100 MHz) has advanced `ticks`: a kernel of known length for
+// streams_at_once, whose every wave ends.
+__global__ void __launch_bounds__(WAVE) hold_kernel(uint64_t ticks) {
+    if (threadIdx.x == 0) {
+        const uint64_t t0 = __builtin_amdgcn_s_memrealtime();
+        while (__builtin_amdgcn_s_memrealtime() - t0 < ticks) __builtin_amdgcn_s_sleep(4);
+    }
+}
+// Whether work on streams a and b runs at once: a 100 us wait on each, released together. One after another they take
+// ~200 us from the release to the later end, at once ~100 us and the launch gap. (Waits for both streams' work first.)
+hipError_t streams_at_once(hipStream_t a, hipStream_t b, bool& at_once) {
+    constexpr uint64_t TICKS = 10000;                   // 100 us
+    hipEvent_t e0 = nullptr, ea = nullptr, eb = nullptr;
+    hipError_t e = hipEventCreate(&e0);
+    if (e == hipSuccess) e = hipEventCreate(&ea);
+    if (e == hipSuccess) e = hipEventCreate(&eb);
+    if (e == hipSuccess) e = hipStreamSynchronize(a);
+    if (e == hipSuccess) e = hipStreamSynchronize(b);
+    if (e == hipSuccess) e = hipEventRecord(e0, a);
+    if (e == hipSuccess) e = hipStreamWaitEvent(b, e0, 0);
+    if (e == hipSuccess) { hipLaunchKernelGGL(hold_kernel, dim3(1), dim3(WAVE), 0, a, TICKS); e = hipGetLastError(); }
+    if (e == hipSuccess) { hipLaunchKernelGGL(hold_kernel, dim3(1), dim3(WAVE), 0, b, TICKS); e = hipGetLastError(); }
+    if (e == hipSuccess) e = hipEventRecord(ea, a);
+    if (e == hipSuccess) e = hipEventRecord(eb, b);
+    if (e == hipSuccess) e = hipEventSynchronize(ea);
+    if (e == hipSuccess) e = hipEventSynchronize(eb);
+    float ta = 0.f, tb = 0.f;
+    if (e == hipSuccess) e = hipEventElapsedTime(&ta, e0, ea);
+    if (e == hipSuccess) e = hipEventElapsedTime(&tb, e0, eb);
+    for (hipEvent_t x : {e0, ea, eb}) if (x) (void)hipEventDestroy(x);
+    at_once = e == hipSuccess && std::max(ta, tb) < 1.5f * 1e-5f * (float)TICKS;
+    return e;
+}
+// A new stream on a hardware queue of its own beside streams a and b (b may be null: a alone), as far as a few tries
+// find one; else the first tried. HIP maps streams onto the process's GPU_MAX_HW_QUEUES queues (4 by default), and
+// kernels of streams that share a queue run one after another: a 65,536-window q16k batch took 642 us in a process
+// whose side streams had queues of their own and 1,041 in one where they had not, 2^28 bases of one haplotype 223 and
+// 334. Above MEASURED_QUEUES the GPU's scheduler shares its queue slots in turns and the test says nothing.
+constexpr int QUEUE_TRIES = 6, MEASURED_QUEUES = 8;
+hipStream_t stream_beside(hipStream_t a, hipStream_t b) {
+    const char* q = getenv("GPU_MAX_HW_QUEUES");
+    const bool measured = !serialised_dispatch() && (!q || atoi(q) <= MEASURED_QUEUES);
+    hipStream_t tried[QUEUE_TRIES];
+    int n = 0, pick = 0;
+    while (n < QUEUE_TRIES) {
+        if (hipStreamCreateWithFlags(&tried[n], hipStreamNonBlocking) != hipSuccess) { (void)hipGetLastError(); break; }
+        n++;
+        bool ok = true;
+        if (measured && (streams_at_once(a, tried[n - 1], ok) != hipSuccess || (ok && b && streams_at_once(b, tried[n - 1], ok) != hipSuccess))) {
+            (void)hipGetLastError();
+            break;
+        }
+        if (ok) { pick = n - 1; break; }
+    }
+    for (int i = 0; i < n; i++) if (i != pick) (void)hipStreamDestroy(tried[i]);
+    return n ? tried[pick] : nullptr;
+}
+
 // A large call's heavy waves run on a second stream beside its light lanes: per launch stream (per device) a side
 // stream and two events, made on the first large call on that stream and kept for the process (at most MAXFORKS
 // launch streams per device; past that, and for callers that must not create streams, the two kernels run one after
@@ -2359,7 +2430,7 @@ const Fork* fork_of(hipStream_t st, bool two = false) {
         if ((int)set.size() >= MAXFORKS) return nullptr;
         if (set.capacity() < (size_t)MAXFORKS) set.reserve(MAXFORKS);       // entries never move
         Fork n{st, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr};
-        if (hipStreamCreateWithFlags(&n.side, hipStreamNonBlocking) != hipSuccess ||
+        if (!(n.side = stream_beside(st, nullptr)) ||
             hipEventCreateWithFlags(&n.fork, hipEventDisableTiming) != hipSuccess ||
             hipEventCreateWithFlags(&n.join, hipEventDisableTiming) != hipSuccess) {
             (void)hipGetLastError();
@@ -2371,7 +2442,7 @@ const Fork* fork_of(hipStream_t st, bool two = false) {
     if (two && !f->side2) {
         hipStream_t s2 = nullptr;
         hipEvent_t lanes = nullptr, join2 = nullptr;
-        if (hipStreamCreateWithFlags(&s2, hipStreamNonBlocking) != hipSuccess ||
+        if (!(s2 = stream_beside(st, f->side)) ||
             hipEventCreateWithFlags(&lanes, hipEventDisableTiming) != hipSuccess ||
             hipEventCreateWithFlags(&join2, hipEventDisableTiming) != hipSuccess) {
             (void)hipGetLastError();
@@ -2843,19 +2914,6 @@ DevSync* sync_of(int dev) {
     }
     return dev_sync[dev];
 }
-// A tool that serialises kernel dispatches (rocprofv3 counter collection or thread trace, which set these variables for
-// the process they profile): a caller wait carried out as a polling kernel would then wait for a lane kernel that
-// cannot start until the poll ends, so the counter wait falls back to events there.
-bool serialised_dispatch() {
-    static const bool on = [] {
-        for (const char* v : {"ROCPROF_COUNTER_COLLECTION", "ROCPROF_COUNTERS", "ROCPROF_COUNTER_GROUPS", "ROCPROF_ADVANCED_THREAD_TRACE"}) {
-            const char* s = getenv(v);
-            if (s && *s && strcmp(s, "0") != 0 && strcasecmp(s, "false") != 0) return true;
-        }
-        return false;
-    }();
-    return on;
-}
 // The marks of stream st in `set` (lanes or callers), created on first use with nev events (with S.mu held); with
 // `counter` (and stream wait-value support) also a counter, zeroed before any wait can read it - signal memory does not
 // start at 0, and a zeroing write only enqueued could land after a first wait had read the old value. nullptr on a HIP
@@ -2917,43 +2975,13 @@ hipError_t sig_mark(Sig& C, bool event) {
 
 extern "C" int32_t pv_dispatch_serialised(void) { return serialised_dispatch() ? 1 : 0; }
 
-namespace {
-// One lane waits until the GPU's real-time clock (100 MHz) has advanced `ticks`: a kernel of known length for
-// pv_streams_concurrent, whose every wave ends.
-__global__ void __launch_bounds__(WAVE) hold_kernel(uint64_t ticks) {
-    if (threadIdx.x == 0) {
-        const uint64_t t0 = __builtin_amdgcn_s_memrealtime();
-        while (__builtin_amdgcn_s_memrealtime() - t0 < ticks) __builtin_amdgcn_s_sleep(4);
-    }
-}
-}  // namespace
-
 extern "C" int32_t pv_streams_concurrent(void* a, void* b, int32_t* concurrent, char* err, size_t errcap) {
     if (!concurrent) { seterr(err, errcap, "null argument"); return PV_EARG; }
     *concurrent = 0;
-    constexpr uint64_t TICKS = 10000;                   // 100 us
-    const hipStream_t sa = (hipStream_t)a, sb = (hipStream_t)b;
-    hipEvent_t e0 = nullptr, ea = nullptr, eb = nullptr;
-    hipError_t e = hipEventCreate(&e0);
-    if (e == hipSuccess) e = hipEventCreate(&ea);
-    if (e == hipSuccess) e = hipEventCreate(&eb);
-    if (e == hipSuccess) e = hipStreamSynchronize(sa);
-    if (e == hipSuccess) e = hipStreamSynchronize(sb);
-    if (e == hipSuccess) e = hipEventRecord(e0, sa);
-    if (e == hipSuccess) e = hipStreamWaitEvent(sb, e0, 0);
-    if (e == hipSuccess) { hipLaunchKernelGGL(hold_kernel, dim3(1), dim3(WAVE), 0, sa, TICKS); e = hipGetLastError(); }
-    if (e == hipSuccess) { hipLaunchKernelGGL(hold_kernel, dim3(1), dim3(WAVE), 0, sb, TICKS); e = hipGetLastError(); }
-    if (e == hipSuccess) e = hipEventRecord(ea, sa);
-    if (e == hipSuccess) e = hipEventRecord(eb, sb);
-    if (e == hipSuccess) e = hipEventSynchronize(ea);
-    if (e == hipSuccess) e = hipEventSynchronize(eb);
-    float ta = 0.f, tb = 0.f;
-    if (e == hipSuccess) e = hipEventElapsedTime(&ta, e0, ea);
-    if (e == hipSuccess) e = hipEventElapsedTime(&tb, e0, eb);
-    for (hipEvent_t x : {e0, ea, eb}) if (x) (void)hipEventDestroy(x);
+    bool at_once = false;
+    const hipError_t e = streams_at_once((hipStream_t)a, (hipStream_t)b, at_once);
     if (e != hipSuccess) { seterr(err, errcap, hipGetErrorString(e)); return PV_EHIP; }
-    // one after another: ~200 us from the release to the later end; at once: ~100 us and the launch gap
-    *concurrent = std::max(ta, tb) < 1.5f * 1e-5f * (float)TICKS ? 1 : 0;
+    *concurrent = at_once ? 1 : 0;
     return PV_OK;
 }
 
