@@ -1507,6 +1507,8 @@ constexpr uint64_t SMALL_SLOTS_Q16 = 2048;
 template <int Q> constexpr uint64_t small_slots() { return Cfg<Q>::REGOPS ? SMALL_SLOTS : SMALL_SLOTS_Q16; }
 // ONE: a call of one window of at most 64 slots (a fetch): its light wave stages the window's assembly's model table in
 // LDS (every slot shares it) before its lanes decode, so that the decode's table reads wait on LDS, not on L2 or HBM.
+// Such a call takes this kernel at Q = 16384 too: a fetch of 5,000 bases 93.5 us by the wave decoder in windows_kernel
+// (65 us of it, after a launch for the coordinates) and 71.6 us by a light lane here (46 us) and the replay (13 us).
 template <int Q, bool ONE = false>
 __global__ void __launch_bounds__(WAVE) front_kernel(pv_dev_cohort D, const int64_t* __restrict__ wasm, const int64_t* __restrict__ wstart,
                                                      uint32_t W, uint32_t bpw, uint64_t nslots, uint8_t* __restrict__ slotbuf, SampleIn X,
@@ -2630,6 +2632,12 @@ static int32_t refuse_capture(hipStream_t st, char* err, size_t errcap) {
     return PV_OK;
 }
 
+static bool capturing(hipStream_t st) {
+    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(st, &cs) != hipSuccess) { (void)hipGetLastError(); return true; }
+    return cs != hipStreamCaptureStatusNone;
+}
+
 // X: the sampler's inputs when light_decode_kernel computes the windows' coordinates (the light path must then be
 // taken: the caller checked light_scratch_bytes), else nullptr
 static int32_t windows_any(const pv_dev_cohort* D, const int64_t* asm_idx, const int64_t* start, int64_t n, int64_t W, const uint8_t* rc,
@@ -2654,9 +2662,8 @@ static int32_t windows_any(const pv_dev_cohort* D, const int64_t* asm_idx, const
     const uint64_t need = light_scratch_bytes(Q, n, W);
     if (work && ((uintptr_t)work & 15)) { seterr(err, errcap, "work buffer not 16-byte aligned"); return PV_EARG; }
     uint8_t* slotbuf = (work && need && work_bytes >= need) ? (uint8_t*)work : nullptr;
-    // a call of one or two slots at Q = 16384 (a fetch) is one block's serial decode: the wave decoder does it and the
-    // replay in one kernel, where the light lanes would add a launch and a slot record's round trip
-    if (Q == 16384 && nslots <= 2 && !X) slotbuf = nullptr;
+    // a call of one or two slots at Q = 16384 that is being captured goes without a work buffer, by the wave decoder
+    if (Q == 16384 && nslots <= 2 && !X && slotbuf && capturing((hipStream_t)stream)) slotbuf = nullptr;
     if (X && !slotbuf) { seterr(err, errcap, "sampler coordinates need the light-block slot records"); return PV_EARG; }
     if (slotbuf) {
         const int32_t cap = refuse_capture((hipStream_t)stream, err, errcap);
@@ -2749,7 +2756,8 @@ extern "C" int32_t pv_fetch_hip(const pv_dev_cohort* D, int64_t assembly, int64_
     if (W < 0 || W >= (1ll << 31)) { seterr(err, errcap, "W"); return PV_EARG; }
     int64_t* R = (int64_t*)rec;
     const uint32_t Q = D->Q;
-    if (W > 0 && Q != 16384 && work && light_scratch_bytes(Q, 1, W) && work_bytes >= light_scratch_bytes(Q, 1, W)) {
+    const bool bare = Q == 16384 && W <= 16384 && capturing((hipStream_t)stream);       // (one or two slots: windows_any)
+    if (W > 0 && !bare && work && light_scratch_bytes(Q, 1, W) && work_bytes >= light_scratch_bytes(Q, 1, W)) {
         // the decode kernel takes the coordinates as arguments and writes the record itself: one launch fewer
         SampleIn X{};
         X.fixed = 1; X.fa = assembly; X.fs = start; X.rcmode = rc ? 1 : 0;
