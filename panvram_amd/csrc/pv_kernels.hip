@@ -359,6 +359,7 @@ struct RefView {
     const uint8_t* g; uint64_t n; int64_t wbase; uint32_t wlen;
     const uint32_t* pw; const int64_t* pes; const int64_t* pel; const uint8_t* peb; const uint32_t* peix; int64_t pne;
 };
+typedef uint32_t v4u __attribute__((ext_vector_type(4)));
 constexpr uint32_t ACGT = 'A' | ('C' << 8) | ('G' << 16) | ('T' << 24);
 // byte q of the packed reference: a run of another byte holding q, else the word's 2-bit code. The bucket index gives
 // the first run ending after the bucket start; runs are sorted and disjoint, so the scan stops at the first run
@@ -370,6 +371,27 @@ __device__ __forceinline__ uint8_t packed_at(const RefView& R, uint64_t q) {
         if (q < rs + (uint64_t)R.pel[r]) return R.peb[r];
     }
     return (uint8_t)(ACGT >> (8 * ((R.pw[q >> 4] >> (2 * (q & 15))) & 3)));
+}
+// bytes [q, q + 16) of the packed reference (all inside it): two words' codes, four to a dword by a byte permute, and the
+// runs of other bytes that overlap them
+__device__ __forceinline__ v4u packed16(const RefView& R, uint64_t q) {
+    const uint32_t c = __builtin_amdgcn_alignbit(R.pw[(q >> 4) + 1], R.pw[q >> 4], 2 * (uint32_t)(q & 15));
+    int64_t r = R.peix[q >> PV_EXC_BUCKET_BITS];
+    v4u v;
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+        const uint32_t x = (c >> (8 * i)) & 0xFF;
+        v[i] = __builtin_amdgcn_perm(0u, ACGT, (x | (x << 6) | (x << 12) | (x << 18)) & 0x03030303u);
+    }
+    for (; r < R.pne; r++) {
+        const uint64_t rs = (uint64_t)R.pes[r], re = rs + (uint64_t)R.pel[r];
+        if (rs >= q + 16) break;
+        const uint32_t b = R.peb[r];
+#pragma unroll
+        for (int i = 0; i < 16; i++)
+            if (q + i >= rs && q + i < re) v[i / 4] = (v[i / 4] & ~(0xFFu << (8 * (i % 4)))) | b << (8 * (i % 4));
+    }
+    return v;
 }
 template <int Q> __device__ __forceinline__ uint8_t ref_at(const Lds<Q>& S, const RefView& R, uint64_t q) {
     const uint64_t k = q - (uint64_t)R.wbase;
@@ -431,7 +453,6 @@ struct Cache {
 // the op list in VGPRs: op k is lane k % 64 of element k / 64 of a register vector, indexed with the wave-uniform k / 64
 // (an indexed register move; NOPR <= 8 for the block sizes that use it)
 typedef uint32_t v8u __attribute__((ext_vector_type(8)));
-typedef uint32_t v4u __attribute__((ext_vector_type(4)));
 // 16 bytes from global memory at any byte address (one 16-byte load)
 __device__ __forceinline__ v4u gload16(const uint8_t* p) {
     v4u v;
@@ -1775,6 +1796,32 @@ __device__ __forceinline__ void process_slot(LS& S, const pv_dev_cohort& D, cons
                 }
                 return;
             }
+            if (R.pw && (kind & 1) && i1 > i0 + 8) {
+                // off the staged span in the packed form: 16 bytes per lane per pass, the destination's first 16-byte
+                // boundary splitting the head off (a byte per lane at a time, each with its own word, bucket and run
+                // reads, took most of the kernel's time where pieces of the assembly are rearranged)
+                const uint64_t top = (uint64_t)src + len - 1;
+                const uint32_t a0 = dst + i0, a1 = dst + i1, b0 = min((a0 + 15) & ~15u, a1);
+                auto one = [&](uint32_t at) {
+                    S.blk[at] = kind == 1 ? ref_at(S, R, (uint64_t)src + (at - dst)) : pvc::comp(ref_at(S, R, top - (at - dst)));
+                };
+                if (l < b0 - a0) one(a0 + l);
+                for (uint32_t q = b0 + 16 * l; q < a1; q += 16 * WAVE) {
+                    const uint32_t off = q - dst;
+                    if (q + 16 <= a1) {
+                        v4u v = packed16(R, kind == 1 ? (uint64_t)src + off : top - off - 15);
+                        if (kind == 3) {
+                            const v4u u = v;
+                            v.x = comp4(__builtin_bswap32(u.w)); v.y = comp4(__builtin_bswap32(u.z));
+                            v.z = comp4(__builtin_bswap32(u.y)); v.w = comp4(__builtin_bswap32(u.x));
+                        }
+                        *(v4u*)&S.blk[q] = v;
+                    } else {
+                        for (uint32_t i = q; i < a1; i++) one(i);
+                    }
+                }
+                return;
+            }
         }
         if (kind == 1) {
             // four bytes per lane in flight per pass
@@ -1873,15 +1920,20 @@ __device__ __forceinline__ void process_slot(LS& S, const pv_dev_cohort& D, cons
             if (kind == 0) { v = lds16((const uint32_t*)S.aux, src + off); return true; }
             if (kind == 1) {
                 const uint64_t so = (uint64_t)src + off - (uint64_t)R.wbase;
-                if (!(so < R.wlen && R.wlen - so >= 20)) return false;
+                if (!(so < R.wlen && R.wlen - so >= 20)) {
+                    if (!R.pw || (uint64_t)src + off + 16 > R.n) return false;
+                    v = packed16(R, (uint64_t)src + off);
+                    return true;
+                }
                 v = lds16((const uint32_t*)S.refw, (uint32_t)so);
                 return true;
             }
             const uint64_t top = (uint64_t)src + len - 1;
             if (top < (uint64_t)off + 15) return false;
             const uint64_t so = top - off - 15 - (uint64_t)R.wbase;
-            if (!(so < R.wlen && R.wlen - so >= 20)) return false;
-            const v4u u = lds16((const uint32_t*)S.refw, (uint32_t)so);
+            const bool in = so < R.wlen && R.wlen - so >= 20;
+            if (!in && !R.pw) return false;
+            const v4u u = in ? lds16((const uint32_t*)S.refw, (uint32_t)so) : packed16(R, top - off - 15);
             v.x = comp4(__builtin_bswap32(u.w)); v.y = comp4(__builtin_bswap32(u.z));
             v.z = comp4(__builtin_bswap32(u.y)); v.w = comp4(__builtin_bswap32(u.x));
             return true;
