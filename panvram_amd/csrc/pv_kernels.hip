@@ -1986,14 +1986,19 @@ __device__ __forceinline__ void process_slot(LS& S, const pv_dev_cohort& D, cons
                     }
                     pv = gload16(pok ? pa : R.g);
                 }
-                if constexpr (!SPAN && NCH <= 4) {
+                if constexpr (!SPAN && (NCH <= 4 || WINB)) {
                     // from HBM (the reference, or the slot record's literal bytes): the 16-byte reads of all (up to
-                    // four) rounds issued before the first is waited for (one round trip per slot, not per round); a
-                    // chunk past the part, or whose bytes a 16-byte read cannot take, reads the reference's first
-                    // bytes instead and is written byte by byte after. (At q16k, eight or sixteen rounds: the registers
-                    // of four in flight cost more workgroups per CU than the round trips they save.)
-                    constexpr uint32_t G = NCH;
-                    for (uint32_t j0 = 0; j0 < nj; j0 += G) {
+                    // four) rounds issued before the first is waited for (one round trip per slot, not per round), of
+                    // two at a time for the window buffer's up to nine rounds; a chunk past the part, or whose bytes a
+                    // 16-byte read cannot take, reads the reference's first bytes instead and is written byte by byte
+                    // after. The loop over groups is unrolled, so that `own` stays in registers named at compile time:
+                    // 69 VGPRs instead of 78 at q4k, 28 waves per CU instead of 24 (65,536 windows on the ring 355 ->
+                    // 328 us a call). The window buffer's replay (W = 5,000): a round at a time 341 us, two 328 (56
+                    // VGPRs), five 336 (84: 20 waves per CU where its LDS allows 24).
+                    constexpr uint32_t G = NCH <= 4 ? NCH : 2;
+#pragma unroll
+                    for (uint32_t j0 = 0; j0 < NCH; j0 += G) {
+                        if (j0 >= nj) break;
                         const uint8_t* ap[G]; uint32_t aw[G], as_[G], ao[G]; bool ok[G];
 #pragma unroll
                         for (uint32_t g = 0; g < G; g++) {
