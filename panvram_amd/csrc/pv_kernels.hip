@@ -21,7 +21,7 @@
 //      the rANS payload and the reference span the block's start diagonal predicts (plus a margin) into LDS;
 //   2. decode the block's symbol stream - the serial part - with the rANS state wave-uniform: a 6-letter context by
 //      a SWAR compare against its row, a 104-letter context by one LDS compare per lane and two ballots, long literal
-//      runs two literals per step (16 lanes test the 16 symbol pairs at once, one v_readlane takes the winner);
+//      runs three literals per step (64 lanes test the 64 symbol triples at once: literal_windows);
 //      literal bytes are gathered one per lane and stored 64 at a time, copies go to an LDS op list;
 //   3. replay the copies the window needs (reference / reverse-complement / overlapping self copies), 64 lanes per op,
 //      reading the staged reference span from LDS (other positions from HBM);
