@@ -233,6 +233,7 @@ __device__ __forceinline__ uint32_t sym_small(Dec& d, const Small& R, uint32_t r
 //    after those, its last bit set to mark their end. With the 12-bit slot in bits 4-15 and x >> 12 in the high half
 //    word, v_sub (half words) gives the slot's place z in the symbol's range, z < freq << 4 is the range check and
 //    v_mad_u32_u16 on the high halves the decode step; one 64-bit shift by 0 or 8 renormalises, and moves the window.
+//    x < 2^16, where the shift is 8, is x >> 12 < 16: 16 less that, not below 0, into byte 1, then at most 8.
 //    One byte is enough for a symbol of frequency 16 or more (x >= 2^16 before it); rarer symbols, and a context's only
 //    one (its frequency does not fit 12 bits), have entries of frequency 0, which no slot is in.
 //  - A window takes at most 24 payload bits. How many it took is the place of the end mark; the next window's low word
@@ -241,38 +242,44 @@ __device__ __forceinline__ uint32_t sym_small(Dec& d, const Small& R, uint32_t r
 //    gives -1, the sign bit of `fail` is set and the loop leaves after that window; the caller decodes again from the
 //    run's start with as many windows as were good, and the nine literals that were not on the general path.
 //  - The index register (the context, which picks A[r] and B[r]) is set per triple around two moves.
+//  - The compiler puts no wait states into assembly, so the order keeps what gfx950 asks for: nothing reads a vcc or SGPR
+//    that a vector instruction wrote less than two instructions before, the cmpx stands between the write of byte 1 and
+//    its use, and four states lie between the last cmpx and the lane reads, one between their source's write and them.
 //
 // What bounds it is one wave's issue: 4 clocks for a 4-byte instruction, 5.6-6.4 for an 8-byte one, and up to 16 more
 // for a scalar instruction within four vector ones of a vector write to SGPRs, vcc or exec, dependent or not; hence the
-// order below (s_ff1 after the two lane reads; mad before cmpx, except in the third literal, whose check the
-// select reads first). Measured on one wave, 4,005 literals (shader clocks a literal): 98.3 with the triple step in C++
+// order below (s_ff1 after the two lane reads; mad before cmpx). Measured on one wave, 4,005 literals (shader clocks a literal): 98.3 with the triple step in C++
 // (63 instructions a triple: two 64-bit shifts per renormalisation, masks in SGPRs, byte counts packed into the
 // state), 82.9 with this step and C++ around three triples, 65.8 with the whole loop in assembly and the shift
 // from leading zeros, 64.5 with it from a compare, 61.1 with v_readfirstlane under the narrowed exec, 59.4 with the
-// scalar work ordered as it is; a window's bookkeeping moved into the next triple's first literal 59.3. In the kernels:
-// front_kernel of sample(1024, 8192) 168 -> 120 us (mean of 13 calls), the longest q16k block 715 -> 450 us.
+// scalar work ordered as it is; a window's bookkeeping moved into the next triple's first literal 59.3. Those from 64.5 on
+// took the shift from a compare and a select that read vcc without its two wait states. What it costs to do without, in
+// us a call of the longest block alone (q4k, 1,030 payload bytes; q16k, 4,104): that form 117.4 and 443.6; two wait
+// states after the compare 131.2 and 497.5; the shift from leading zeros (three instructions) 124.5 and 466.5; as it is
+// 120.7 and 446.5.
 typedef uint32_t v16u __attribute__((ext_vector_type(16)));
 constexpr uint32_t LIT_WIN = 9, LIT_RUN = 21;      // literals per window; windows per run (3 bytes each: words' 64 lanes)
 #define PV_LIT_STEP(src, e) \
     "v_sub_u32_sdwa %[z], " src ", " e " dst_sel:DWORD dst_unused:UNUSED_PAD src0_sel:WORD_0 src1_sel:WORD_0\n"
 #define PV_LIT_MAD(src, e) "v_mad_u32_u16 v97, " src ", " e ", %[z] op_sel:[1,1,0,0]\n"
 #define PV_LIT_CHECK(e) "v_cmpx_lt_u32_sdwa vcc, %[z], " e " src0_sel:DWORD src1_sel:WORD_1\n"
-#define PV_LIT_NORM "v_cmp_gt_u32 vcc, %[low], v97\n" "v_cndmask_b32 %[z], 0, %[eight], vcc\n" "v_lshlrev_b64 v[96:97], %[z], v[96:97]\n"
+#define PV_LIT_LOW "v_sub_u32_sdwa %[s], %[sixteen], v97 clamp dst_sel:BYTE_1 dst_unused:UNUSED_PAD src0_sel:DWORD src1_sel:WORD_1\n"
+#define PV_LIT_NORM "v_min_u32 %[s], 8, %[s]\n" "v_lshlrev_b64 v[96:97], %[s], v[96:97]\n"
 // the context's entries (acc's low four bits; idx: the register they are put in), then the triple and its select
 #define PV_LIT_TRIPLE(idx) \
     "s_and_b32 " idx ", %[acc], 15\n" "s_set_gpr_idx_on " idx ", gpr_idx(SRC0)\n" "v_mov_b32 %[a], v64\n" "v_mov_b32 %[b], v80\n" \
     "s_set_gpr_idx_off\n" "v_mov_b32 v96, %[lo]\n" \
-    PV_LIT_STEP("%[y]", "%[a]") PV_LIT_MAD("%[y]", "%[a]") PV_LIT_CHECK("%[a]") PV_LIT_NORM \
-    PV_LIT_STEP("v97", "%[b]") PV_LIT_MAD("v97", "%[b]") PV_LIT_CHECK("%[b]") PV_LIT_NORM \
-    PV_LIT_STEP("v97", "%[c]") PV_LIT_CHECK("%[c]") PV_LIT_MAD("v97", "%[c]") PV_LIT_NORM \
-    "s_nop 0\n" "v_readfirstlane_b32 %[lo], v96\n" "v_readfirstlane_b32 %[y], v97\n" "s_ff1_i32_b64 %[t], exec\n" \
+    PV_LIT_STEP("%[y]", "%[a]") PV_LIT_MAD("%[y]", "%[a]") PV_LIT_LOW PV_LIT_CHECK("%[a]") PV_LIT_NORM \
+    PV_LIT_STEP("v97", "%[b]") PV_LIT_MAD("v97", "%[b]") PV_LIT_LOW PV_LIT_CHECK("%[b]") PV_LIT_NORM \
+    PV_LIT_STEP("v97", "%[c]") PV_LIT_MAD("v97", "%[c]") PV_LIT_LOW PV_LIT_CHECK("%[c]") PV_LIT_NORM \
+    "s_nop 1\n" "v_readfirstlane_b32 %[lo], v96\n" "v_readfirstlane_b32 %[y], v97\n" "s_ff1_i32_b64 %[t], exec\n" \
     "s_lshl_b32 %[acc], %[acc], 6\n" "s_mov_b64 exec, %[ex]\n" "s_or_b32 %[acc], %[acc], %[t]\n"
 // y: x << 4 | the next 4 payload bits; r: the context; words: as above; n: windows (1 .. LIT_RUN), all lanes the same.
 // Returns in lane i of `lits` window i's context and literals (4 + 18 bits, the first literal's highest), in y, r and
 // bits the state after the last window, in n the windows done, the last of them not good when fail is negative.
 __device__ __forceinline__ void literal_windows(uint32_t& y, uint32_t& r, uint32_t& n, uint32_t& bits, int32_t& fail, uint32_t& lits,
                                                 uint32_t words, const v16u& A, const v16u& B, uint32_t C) {
-    uint32_t yy = rfl(y), acc = rfl(r), lo = rdl(words, 0), k = 0, P = 0, t, i, z, a, b, m; int32_t f; uint64_t ex;
+    uint32_t yy = rfl(y), acc = rfl(r), lo = rdl(words, 0), k = 0, P = 0, t, i, z, s, a, b, m; int32_t f; uint64_t ex;
     const uint32_t end = rfl(n);
     asm volatile(
         "s_mov_b64 %[ex], exec\n"
@@ -294,14 +301,15 @@ __device__ __forceinline__ void literal_windows(uint32_t& y, uint32_t& r, uint32
         "s_mov_b32 m0, %[m]\n"
         "s_nop 1\n"
         : [y] "+&s"(yy), [lo] "+&s"(lo), [acc] "+&s"(acc), [k] "+&s"(k), [P] "+&s"(P), [lits] "+&v"(lits), [t] "=&s"(t), [i] "=&s"(i), [f] "=&s"(f),
-          [ex] "=&s"(ex), [m] "=&s"(m), [z] "=&v"(z), [a] "=&v"(a), [b] "=&v"(b)
-        : "{v[64:79]}"(A), "{v[80:95]}"(B), [c] "v"(C), [words] "v"(words), [end] "s"(end), [low] "s"(0x100000u), [eight] "v"(8u)
+          [ex] "=&s"(ex), [m] "=&s"(m), [z] "=&v"(z), [s] "=&v"(s), [a] "=&v"(a), [b] "=&v"(b)
+        : "{v[64:79]}"(A), "{v[80:95]}"(B), [c] "v"(C), [words] "v"(words), [end] "s"(end), [sixteen] "v"(16u)
         : "v96", "v97", "vcc", "scc");
     y = rfl(yy); r = rfl(acc) & 15; n = rfl(k); bits = rfl(P); fail = (int32_t)rfl((uint32_t)f);
 }
 #undef PV_LIT_STEP
 #undef PV_LIT_MAD
 #undef PV_LIT_CHECK
+#undef PV_LIT_LOW
 #undef PV_LIT_NORM
 #undef PV_LIT_TRIPLE
 
