@@ -195,7 +195,9 @@ typedef struct pv_dev_cohort {
  * Launches on `stream` (a hipStream_t; NULL = the null stream) and returns without waiting.
  * work / work_bytes: optional device scratch (16-byte aligned). With at least pv_windows_work_bytes(D, n, W) bytes,
  * blocks with short payloads are decoded one lane per block by a first kernel and the windows kernel only replays
- * them; with less (or NULL) every block is decoded by the windows kernel. The bytes returned are the same.
+ * them; with less (or NULL) every block is decoded by the windows kernel. The bytes returned are the same. A buffer is
+ * for one call at a time: calls that follow each other on one stream may share it, calls issued by several threads may
+ * not, also on one stream (a call's launches pass records through it, and another thread's may come between them).
  * Replaces _C.windows_cuda / pv_windows_cuda + run_windows (reference csrc/pv_cuda.cu:117-162), including its checks:
  * Q in {1024, 2048, 4096, 16384}, 0 <= W < 2^31, n * (ceil(W/Q)+1) < 2^31 -> PV_EARG.
  * A call that uses the work buffer refuses a stream under graph capture (PV_EARG): its list and done words carry a

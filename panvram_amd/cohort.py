@@ -293,8 +293,9 @@ class Cohort:
         self._callers = {}            # (stream id, device, type) -> torch Stream of a caller's current stream
         self._sample_args = {}        # W -> the constant pointer arguments of pv_sample_hip
         self._work_bytes = {}         # (n, W, light) -> bytes of pv_sample_hip's work
-        # per stream: the device buffer its decode calls use for work, draws and status. Calls on one stream run in
+        # per stream: the device buffer its `sample` calls use for work, draws and status. Calls on one stream run in
         # order, so each reuses the buffer of the one before (no allocation per call); grown when a call needs more.
+        # (`fetch` and `windows` keep one per thread and stream: _thread_buffer.)
         self._stream_work = {}
         self._views = {}              # (stream, buffer, n, work bytes, rc mode) -> views of draws, uniforms, status
         self._err = N.errbuf()        # the C calls' error text (written only on failure)
@@ -305,7 +306,7 @@ class Cohort:
         self._plans = {}              # assembly -> FASTA layout plan (check_full)
         self._aux = None              # the stream check_full and decode() decode on
         self._aux2 = None             # the two streams decode() copies to the host on
-        self._local = threading.local()   # per thread: fetch()'s 32-byte coordinate record on the device
+        self._local = threading.local()   # per thread: fetch()'s 32-byte record on the device, the work buffers by stream
 
     def _upload(self):
         L = N.lib()
@@ -452,7 +453,7 @@ class Cohort:
         return out, status
 
     def _stream_buffer(self, key, nbytes):
-        """The work buffer of the stream with handle `key` (the current stream), at least nbytes."""
+        """`sample`'s work buffer of the stream with handle `key` (the current stream), at least nbytes."""
         buf = self._stream_work.get(key)
         if buf is None or buf.numel() < nbytes:
             if len(self._stream_work) >= 64:
@@ -465,12 +466,27 @@ class Cohort:
             buf = self._stream_work[key] = torch.empty(nbytes, dtype=torch.uint8, device=self.device)
         return buf
 
+    def _thread_buffer(self, key, nbytes):
+        """The calling thread's work buffer for `fetch` and `windows` on the stream with handle `key`, at least nbytes.
+        A call is two or more launches that pass slot records through it, and ctypes drops the GIL between them: with one
+        buffer per stream, two threads on one stream (torch's default stream is the same for all) would replay each
+        other's records. Freed with the thread or the cohort, like every torch tensor after its stream's work."""
+        work = getattr(self._local, "work", None)
+        if work is None:
+            work = self._local.work = {}
+        buf = work.get(key)
+        if buf is None or buf.numel() < nbytes:
+            if len(work) >= 64:
+                work.clear()
+            buf = work[key] = torch.empty(nbytes, dtype=torch.uint8, device=self.device)
+        return buf
+
     def _windows_into(self, asm, start, W, rc, tokens, apply_case, out, status, ids=None):
         err, ev = N.errbuf(), self.kernel_events
         with torch.cuda.device(self.device):
             stream = torch.cuda.current_stream(self.device).cuda_stream
             wb = int(N.lib().pv_windows_work_bytes(ctypes.byref(self._D), asm.numel(), W)) if self.light_decode else 0
-            wp = self._stream_buffer(stream, wb).data_ptr() if wb else None
+            wp = self._thread_buffer(stream, wb).data_ptr() if wb else None
             if ev is not None:
                 t0, t1 = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
                 t0.record()
@@ -840,7 +856,7 @@ class Cohort:
         err, L, D = loc.err, N.lib(), self._Dref
         stream = torch.cuda.current_stream(dev).cuda_stream
         wb = int(L.pv_windows_work_bytes(D, 1, length)) if self.light_decode else 0
-        wp = self._stream_buffer(stream, wb).data_ptr() if wb else None
+        wp = self._thread_buffer(stream, wb).data_ptr() if wb else None
         args = (D, a, boff + start, length, int(bool(reverse_complement)), int(bool(tokens)), out.data_ptr(), rec.data_ptr(), wp, wb,
                 stream, err, len(err))
         ev = self.kernel_events

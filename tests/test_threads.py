@@ -1,0 +1,88 @@
+"""Calls from several threads on one stream: a `fetch` or `windows` call passes slot records from one launch to the next
+through a work buffer, so each thread has its own."""
+import threading
+import types
+
+import numpy as np
+import pytest
+import torch
+
+from oracle import oracle as O
+
+
+def test_each_thread_has_its_work_buffer(monkeypatch):
+    """Two threads on one stream: the work pointers given to the library differ, and each thread's stays the same."""
+    from panvram_amd import cohort as M
+    calls = []
+
+    class Lib:
+        def pv_windows_work_bytes(self, D, n, W):
+            return 1536
+
+        def pv_fetch_hip(self, *a):
+            calls.append((threading.get_ident(), a[8]))
+            return 0
+
+    lib = Lib()
+    monkeypatch.setattr(M.N, "lib", lambda: lib)
+    monkeypatch.setattr(torch.cuda, "current_stream", lambda *a: types.SimpleNamespace(cuda_stream=0))
+    monkeypatch.setattr(torch.cuda, "current_device", lambda: 0)
+    c = M.Cohort.__new__(M.Cohort)
+    c.names, c._by_name, c._ctgs, c._ctg_index = ["a"], {"a": 0}, [[("c", "c", 1000, 0, 60)]], [{"c": 0}]
+    c.device, c._idx, c._Dref, c._h, c.light_decode, c.kernel_events = torch.device("cpu"), 0, None, None, True, None
+    c._local, c._stream_work, c._views, c._fast = threading.local(), {}, {}, {}
+    meet, failed = threading.Barrier(2), []
+
+    def work():
+        try:
+            for _ in range(2):
+                c.fetch(0, 0, 5, 100)
+                meet.wait(30)                                      # both are alive at every call
+        except Exception as e:
+            failed.append(e)
+            meet.abort()
+
+    ts = [threading.Thread(target=work) for _ in range(2)]
+    [t.start() for t in ts]
+    [t.join() for t in ts]
+    assert not failed, failed
+    by = {}
+    for who, ptr in calls:
+        by.setdefault(who, set()).add(ptr)
+    a, b = by.values()
+    assert len(a) == len(b) == 1 and None not in a | b and a != b
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("ds", ["q1k", "q4k", "q16k"])
+def test_threads_on_one_stream_equal_oracle(fx, oracle_ref, ds):
+    """Four threads on the default stream, each with lengths of its own and `fetch` and `windows` in turn."""
+    import panvram_amd
+    c = panvram_amd.Cohort.open(fx["dirs"][ds], device="cuda", dataset=ds, reference=fx["ref"])
+    arcs = [O.Archive(f"{fx['dirs'][ds]}/{nm}.{ds}.rr3") for nm in c.names]
+    full = [A.full(oracle_ref) for A in arcs]
+    bad = []
+
+    def work(t):
+        try:
+            rng = np.random.default_rng(100 + t)
+            W = (37, 1500, 5000, 16000)[t]
+            for k in range(150):
+                a = int(rng.integers(len(c)))
+                rows = [(i, x) for i, x in enumerate(c.contigs(a)) if x[2] >= W]
+                i, x = rows[int(rng.integers(len(rows)))]
+                s = int(rng.integers(x[2] - W + 1))
+                want = full[a][x[3] + s:x[3] + s + W]
+                if k % 3:
+                    got = c.fetch(a, i, s, W).cpu().numpy()
+                else:
+                    got = c.windows(torch.tensor([a]), torch.tensor([x[3] + s]), W)[0].cpu().numpy()
+                if not np.array_equal(got, want):
+                    bad.append((t, k, a, i, s, W))
+        except Exception as e:
+            bad.append((t, repr(e)))
+
+    ts = [threading.Thread(target=work, args=(t,)) for t in range(4)]
+    [t.start() for t in ts]
+    [t.join() for t in ts]
+    assert not bad, bad[:5]
