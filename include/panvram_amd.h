@@ -231,7 +231,8 @@ uint64_t pv_windows_work_bytes(const pv_dev_cohort* D, int64_t n, int64_t W);
  * needs to start at zero, so no call clears it. PV_EARG when n windows of W bases need more than
  * PV_NOALLOC_SCRATCH_BYTES of light-block slots (768 bytes per window x covering block: 43,690 slots, e.g. n = 14,563
  * at W = 8192, q4k); at Q = 16384 such a call runs with no scratch instead (every block by the windows kernel's wave
- * decoder). Other arguments, results and errors as pv_windows_hip. */
+ * decoder), and so does one of one or two window x block slots (n = 1, W <= 16384): such calls may overlap, and be
+ * captured. Other arguments, results and errors as pv_windows_hip. */
 #define PV_NOALLOC_SCRATCH_BYTES (32u << 20)
 int32_t pv_windows_hip_noalloc(const pv_dev_cohort* D, const int64_t* asm_idx, const int64_t* start, int64_t n, int64_t W,
                                const uint8_t* rc, int32_t tokens, int32_t apply_case, uint8_t* out, int32_t* status,

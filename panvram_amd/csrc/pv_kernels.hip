@@ -2863,7 +2863,9 @@ extern "C" int32_t pv_windows_hip_noalloc(const pv_dev_cohort* D, const int64_t*
     if (!D) { seterr(err, errcap, "null argument"); return PV_EARG; }
     const uint32_t Q = D->Q;
     uint64_t need = (W > 0 && W < (1ll << 31) && n > 0 && (uint64_t)n < (1ull << 31)) ? light_scratch_bytes(Q, n, W) : 0;
-    if (need > PV_NOALLOC_SCRATCH_BYTES && Q == 16384) need = 0;   // the wave decoder alone, which needs no scratch
+    // at Q = 16384 the wave decoder alone, which needs no scratch: past the array, and for one or two slots, so that such
+    // calls (single slices) on several streams at once share nothing
+    if (Q == 16384 && (need > PV_NOALLOC_SCRATCH_BYTES || need <= 2 * SLOT_BYTES)) need = 0;
     if (need > PV_NOALLOC_SCRATCH_BYTES) {
         char m[256];
         snprintf(m, sizeof m, "pv_windows_hip_noalloc: %llu windows of %lld bases need %llu bytes of scratch, over the %u this entry "

@@ -86,3 +86,29 @@ def test_threads_on_one_stream_equal_oracle(fx, oracle_ref, ds):
     [t.start() for t in ts]
     [t.join() for t in ts]
     assert not bad, bad[:5]
+
+
+@pytest.mark.gpu
+def test_noalloc_short_q16k_calls_share_nothing(fx, oracle_ref):
+    """pv_windows_hip_noalloc at q16k with one window of at most a block, on three streams at once: no call uses the
+    scratch array, so each row is its own."""
+    import panvram_amd
+    from panvram_amd import _native as N
+    c = panvram_amd.Cohort.open(fx["dirs"]["q16k"], device="cuda", dataset="q16k", reference=fx["ref"])
+    full = [O.Archive(f"{fx['dirs']['q16k']}/{nm}.q16k.rr3").full(oracle_ref) for nm in c.names]
+    rng = np.random.default_rng(9)
+    calls = []
+    for k in range(90):
+        a, W = int(rng.integers(len(c))), (1, 700, 16384)[k % 3]
+        s = int(rng.integers(len(full[a]) - W + 1))
+        calls.append((a, s, W, torch.tensor([a], device="cuda"), torch.tensor([s], device="cuda"),
+                      torch.empty((1, W), dtype=torch.uint8, device="cuda"), torch.zeros(1, dtype=torch.int32, device="cuda")))
+    streams = [torch.cuda.Stream() for _ in range(3)]
+    torch.cuda.synchronize()
+    err = N.errbuf()
+    for k, (a, s, W, ta, ts, out, status) in enumerate(calls):
+        assert N.lib().pv_windows_hip_noalloc(c._Dref, ta.data_ptr(), ts.data_ptr(), 1, W, None, 0, 1, out.data_ptr(), status.data_ptr(),
+                                              streams[k // 3 % 3].cuda_stream, err, len(err)) == 0, err.value
+    torch.cuda.synchronize()
+    for a, s, W, _, _, out, status in calls:
+        assert int(status) == 0 and np.array_equal(out[0].cpu().numpy(), full[a][s:s + W]), (a, s, W)
