@@ -206,12 +206,15 @@ int32_t pv_windows_hip(const pv_dev_cohort* D, const int64_t* asm_idx, const int
                        const uint8_t* rc, int32_t tokens, int32_t apply_case, uint8_t* out, int32_t* status,
                        void* work, uint64_t work_bytes, void* stream, char* err, size_t errcap);
 /* What a call of n windows of W bases on `stream` uses besides its buffers, set up ahead of the first such call: for a
- * call of more than 16,384 (window, covering block) slots (2,048 at Q = 16384), the side stream its long-block decode runs on (the heavy
- * waves at Q <= 4096; at Q = 16384 the whole-slot pass, beside the replay) and the two events that fork and join it
- * (otherwise made by the first such call on the stream). pv_windows_hip and
- * pv_sample_hip on the caller's own stream fork; pv_sample_hip on a ring stream does not (the ring overlaps calls). Idempotent; PV_OK
- * also where nothing is needed or the side stream cannot be had (such calls then run on `stream` alone). Call with
- * the stream's device current. No reference counterpart. */
+ * call of more than 16,384 (window, covering block) slots (2,048 at Q = 16384), the side stream its long-block decode runs
+ * on (the heavy waves at Q <= 4096; at Q = 16384 the whole-slot pass, and a second one for the replay) and the events that
+ * fork and join it (otherwise made by the first such call on the stream). At up to 8 hardware queues one of the first
+ * calls that finds the stream run dry, this one or a large call, also tries whether the side streams run beside it, with
+ * waits of 100 us on both, and replaces those that do not: a few milliseconds of host time once per stream. Nothing here,
+ * nor in a decode call, waits for work queued on the stream: where it is busy the trial is left to a later call (four at
+ * most). pv_windows_hip and pv_sample_hip on the caller's own stream fork; pv_sample_hip on a ring stream does not (the
+ * ring overlaps calls). Idempotent; PV_OK also where nothing is needed or the side stream cannot be had (such calls then
+ * run on `stream` alone). Call with the stream's device current. No reference counterpart. */
 int32_t pv_launch_prepare(const pv_dev_cohort* D, int64_t n, int64_t W, void* stream, char* err, size_t errcap);
 /* Host check of the decode kernels' four-bytes-at-a-time output transforms (complement, complement keeping case,
  * token codes, lower-case flags) against their per-byte definitions, over every byte value: the number of mismatches

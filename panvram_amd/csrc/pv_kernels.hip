@@ -2419,23 +2419,37 @@ __global__ void __launch_bounds__(WAVE) hold_kernel(uint64_t ticks) {
     }
 }
 // Whether work on streams a and b runs at once: a 100 us wait on each, released together. One after another they take
-// ~200 us from the release to the later end, at once ~100 us and the launch gap. (Waits for both streams' work first.)
-hipError_t streams_at_once(hipStream_t a, hipStream_t b, bool& at_once) {
+// ~200 us from the release to the later end, at once ~100 us and the launch gap. may_wait: waits for both streams' work
+// first, however long. Else it waits for nothing that is queued there: hipErrorNotReady when the streams have not run
+// dry within TRIAL_IDLE_S, or the two waits not ended within TRIAL_S (work that came between on a busy GPU).
+constexpr double TRIAL_IDLE_S = 1e-3, TRIAL_S = 2e-3;
+hipError_t streams_at_once(hipStream_t a, hipStream_t b, bool& at_once, bool may_wait) {
     constexpr uint64_t TICKS = 10000;                   // 100 us
+    auto until = [](double limit, auto&& query) {
+        const auto t0 = std::chrono::steady_clock::now();
+        for (;;) {
+            const hipError_t e = query();
+            if (e != hipErrorNotReady) return e;
+            (void)hipGetLastError();
+            if (std::chrono::duration<double>(std::chrono::steady_clock::now() - t0).count() > limit) return e;
+        }
+    };
+    auto dry = [&](hipStream_t s) { return may_wait ? hipStreamSynchronize(s) : until(TRIAL_IDLE_S, [&] { return hipStreamQuery(s); }); };
+    auto ended = [&](hipEvent_t x) { return may_wait ? hipEventSynchronize(x) : until(TRIAL_S, [&] { return hipEventQuery(x); }); };
     hipEvent_t e0 = nullptr, ea = nullptr, eb = nullptr;
     hipError_t e = hipEventCreate(&e0);
     if (e == hipSuccess) e = hipEventCreate(&ea);
     if (e == hipSuccess) e = hipEventCreate(&eb);
-    if (e == hipSuccess) e = hipStreamSynchronize(a);
-    if (e == hipSuccess) e = hipStreamSynchronize(b);
+    if (e == hipSuccess) e = dry(a);
+    if (e == hipSuccess) e = dry(b);
     if (e == hipSuccess) e = hipEventRecord(e0, a);
     if (e == hipSuccess) e = hipStreamWaitEvent(b, e0, 0);
     if (e == hipSuccess) { hipLaunchKernelGGL(hold_kernel, dim3(1), dim3(WAVE), 0, a, TICKS); e = hipGetLastError(); }
     if (e == hipSuccess) { hipLaunchKernelGGL(hold_kernel, dim3(1), dim3(WAVE), 0, b, TICKS); e = hipGetLastError(); }
     if (e == hipSuccess) e = hipEventRecord(ea, a);
     if (e == hipSuccess) e = hipEventRecord(eb, b);
-    if (e == hipSuccess) e = hipEventSynchronize(ea);
-    if (e == hipSuccess) e = hipEventSynchronize(eb);
+    if (e == hipSuccess) e = ended(ea);
+    if (e == hipSuccess) e = ended(eb);
     float ta = 0.f, tb = 0.f;
     if (e == hipSuccess) e = hipEventElapsedTime(&ta, e0, ea);
     if (e == hipSuccess) e = hipEventElapsedTime(&tb, e0, eb);
@@ -2443,29 +2457,37 @@ hipError_t streams_at_once(hipStream_t a, hipStream_t b, bool& at_once) {
     at_once = e == hipSuccess && std::max(ta, tb) < 1.5f * 1e-5f * (float)TICKS;
     return e;
 }
-// A new stream on a hardware queue of its own beside streams a and b (b may be null: a alone), as far as a few tries
-// find one; else the first tried. HIP maps streams onto the process's GPU_MAX_HW_QUEUES queues (4 by default), and
-// kernels of streams that share a queue run one after another: a 65,536-window q16k batch took 642 us in a process
-// whose side streams had queues of their own and 1,041 in one where they had not, 2^28 bases of one haplotype 223 and
-// 334. Above MEASURED_QUEUES the GPU's scheduler shares its queue slots in turns and the test says nothing.
-constexpr int QUEUE_TRIES = 6, MEASURED_QUEUES = 8;
-hipStream_t stream_beside(hipStream_t a, hipStream_t b) {
-    const char* q = getenv("GPU_MAX_HW_QUEUES");
-    const bool measured = !serialised_dispatch() && (!q || atoi(q) <= MEASURED_QUEUES);
-    hipStream_t tried[QUEUE_TRIES];
-    int n = 0, pick = 0;
-    while (n < QUEUE_TRIES) {
-        if (hipStreamCreateWithFlags(&tried[n], hipStreamNonBlocking) != hipSuccess) { (void)hipGetLastError(); break; }
-        n++;
-        bool ok = true;
-        if (measured && (streams_at_once(a, tried[n - 1], ok) != hipSuccess || (ok && b && streams_at_once(b, tried[n - 1], ok) != hipSuccess))) {
+// A stream on a hardware queue of its own beside streams a and b (b may be null: a alone): `have` if it is one, else the
+// first of a few new ones that is; `have` when none is found or nothing can be tried now, with found = false. HIP maps
+// streams onto the process's GPU_MAX_HW_QUEUES queues (4 by default), and kernels of streams that share a queue run one
+// after another: a 65,536-window q16k batch took 642 us in a process whose side streams had queues of their own and
+// 1,041 in one where they had not, 2^28 bases of one haplotype 223 and 334. It runs inside a call that must not wait for
+// what the caller has queued, so it gives up where that is not done soon (streams_at_once), and in this thread's relaxed
+// capture mode, so that its queries do not end a capture of another thread.
+constexpr int QUEUE_TRIES = 6;
+hipStream_t stream_beside(hipStream_t a, hipStream_t b, hipStream_t have, bool& found) {
+    found = false;
+    hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+    if (hipThreadExchangeStreamCaptureMode(&mode) != hipSuccess) { (void)hipGetLastError(); return have; }
+    hipStream_t made[QUEUE_TRIES], pick = have, s = have;
+    int n = 0;
+    for (;;) {
+        bool ok = false;
+        hipError_t e = streams_at_once(a, s, ok, false);
+        if (e == hipSuccess && ok && b) e = streams_at_once(b, s, ok, false);
+        if (e != hipSuccess) {
             (void)hipGetLastError();
+            if (n) n--;                                 // s may hold a wait that is not done: destroying it would wait too
             break;
         }
-        if (ok) { pick = n - 1; break; }
+        if (ok) { found = true; pick = s; break; }
+        if (n == QUEUE_TRIES - 1) break;
+        if (hipStreamCreateWithFlags(&s, hipStreamNonBlocking) != hipSuccess) { (void)hipGetLastError(); break; }
+        made[n++] = s;
     }
-    for (int i = 0; i < n; i++) if (i != pick) (void)hipStreamDestroy(tried[i]);
-    return n ? tried[pick] : nullptr;
+    for (int i = 0; i < n; i++) if (made[i] != pick) (void)hipStreamDestroy(made[i]);
+    (void)hipThreadExchangeStreamCaptureMode(&mode);
+    return pick;
 }
 
 // A large call's heavy waves run on a second stream beside its light lanes: per launch stream (per device) a side
@@ -2479,29 +2501,41 @@ hipStream_t stream_beside(hipStream_t a, hipStream_t b) {
 #ifndef PV_LITE
 #define PV_LITE 1
 #endif
-constexpr int MAXFORKS = 64;
-struct Fork { hipStream_t st, side, side2; hipEvent_t fork, join, lanes, join2; };
+// The side streams are first as they come. One of the next FORK_TRIALS large calls that finds the launch stream dry, or
+// about to be, tries them and replaces those that share its queue (stream_beside: a few milliseconds, outside fork_mu); a
+// call that finds it busy goes on with those there are. A replaced stream is kept, since another thread's call may be
+// using it. Above MEASURED_QUEUES hardware queues the GPU's scheduler shares its queue slots in turns and a trial says
+// nothing.
+constexpr int MAXFORKS = 64, FORK_TRIALS = 4, MEASURED_QUEUES = 8;
+struct Fork { hipStream_t st, side, side2; hipEvent_t fork, join, lanes, join2; bool beside, beside2, trying; int trials; };
 std::mutex fork_mu;
 std::vector<Fork> fork_set[64];
-// The side stream(s) and events of caller stream st, made on first use: the second side stream (two = true, for the
-// whole-slot passes at Q = 16384) only where asked for, since every stream takes one of the process's hardware queues.
-// nullptr when they cannot be had (the call then runs on st alone).
-const Fork* fork_of(hipStream_t st, bool two = false) {
+// Whether streams can be tried at all: not where dispatches are serialised, nor above MEASURED_QUEUES queues
+bool trials_tell() {
+    const char* q = getenv("GPU_MAX_HW_QUEUES");
+    return !serialised_dispatch() && (!q || atoi(q) <= MEASURED_QUEUES);
+}
+// The side stream(s) and events of caller stream st into `out`, made on first use: the second side stream (two = true,
+// for the whole-slot passes at Q = 16384) only where asked for, since every stream takes one of the process's hardware
+// queues. False when they cannot be had (the call then runs on st alone).
+bool fork_of(hipStream_t st, bool two, Fork& out) {
     int dev = 0;
-    if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) { (void)hipGetLastError(); return nullptr; }
-    std::lock_guard<std::mutex> g(fork_mu);
+    if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) { (void)hipGetLastError(); return false; }
+    std::unique_lock<std::mutex> g(fork_mu);
     std::vector<Fork>& set = fork_set[dev];
     Fork* f = nullptr;
     for (Fork& x : set) if (x.st == st) { f = &x; break; }
     if (!f) {
-        if ((int)set.size() >= MAXFORKS) return nullptr;
+        if ((int)set.size() >= MAXFORKS) return false;
         if (set.capacity() < (size_t)MAXFORKS) set.reserve(MAXFORKS);       // entries never move
-        Fork n{st, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr};
-        if (!(n.side = stream_beside(st, nullptr)) ||
+        Fork n{};
+        n.st = st;
+        n.trials = trials_tell() ? FORK_TRIALS : 0;
+        if (hipStreamCreateWithFlags(&n.side, hipStreamNonBlocking) != hipSuccess ||
             hipEventCreateWithFlags(&n.fork, hipEventDisableTiming) != hipSuccess ||
             hipEventCreateWithFlags(&n.join, hipEventDisableTiming) != hipSuccess) {
             (void)hipGetLastError();
-            return nullptr;                                               // (what was made is kept: a few handles)
+            return false;                                                 // (what was made is kept: a few handles)
         }
         set.push_back(n);
         f = &set.back();
@@ -2509,15 +2543,36 @@ const Fork* fork_of(hipStream_t st, bool two = false) {
     if (two && !f->side2) {
         hipStream_t s2 = nullptr;
         hipEvent_t lanes = nullptr, join2 = nullptr;
-        if (!(s2 = stream_beside(st, f->side)) ||
+        if (hipStreamCreateWithFlags(&s2, hipStreamNonBlocking) != hipSuccess ||
             hipEventCreateWithFlags(&lanes, hipEventDisableTiming) != hipSuccess ||
             hipEventCreateWithFlags(&join2, hipEventDisableTiming) != hipSuccess) {
             (void)hipGetLastError();
-            return nullptr;
+            return false;
         }
         f->lanes = lanes; f->join2 = join2; f->side2 = s2;                // (side2 last: it marks the three made)
+        if (trials_tell()) f->trials = FORK_TRIALS;
     }
-    return f;
+    if (f->trials > 0 && !f->trying && (!f->beside || (two && !f->beside2))) {
+        f->trials--;
+        f->trying = true;
+        Fork t = *f;
+        g.unlock();
+        // (a new side stream takes a join event of its own: a call of another thread may be about to wait for the old one's)
+        auto replace = [&](hipStream_t b, hipStream_t& side, hipEvent_t& join, bool& beside) {
+            const hipStream_t x = stream_beside(st, b, side, beside);
+            hipEvent_t e = nullptr;
+            if (x == side) return;
+            if (hipEventCreateWithFlags(&e, hipEventDisableTiming) == hipSuccess) { side = x; join = e; }
+            else { (void)hipGetLastError(); beside = false; }
+        };
+        if (!t.beside) replace(nullptr, t.side, t.join, t.beside);
+        if (t.beside && two && !t.beside2) replace(t.side, t.side2, t.join2, t.beside2);
+        g.lock();
+        f->side = t.side; f->join = t.join; f->beside = t.beside; f->trying = false;
+        if (two) { f->side2 = t.side2; f->join2 = t.join2; f->beside2 = t.beside2; }
+    }
+    out = *f;
+    return true;
 }
 
 template <int Q>
@@ -2526,6 +2581,7 @@ hipError_t launch(const pv_dev_cohort& D, const int64_t* wa, const int64_t* ws, 
                   const SampleIn& X, hipEvent_t ev_mid, hipEvent_t ev_end, hipStream_t st, bool may_fork) {
     bool dec = true;                                    // windows_kernel with the wave decoder
     uint32_t xshift = ~0u;
+    Fork sides{};
     const Fork* fs = nullptr;                           // spill_kernel's list part and windows_kernel on side streams
     const Fork* fh = nullptr;                           // heavy_kernel on a side stream, joined after windows_kernel
     if (slotbuf && (nslots <= small_slots<Q>() || !HL.cap)) {
@@ -2544,7 +2600,7 @@ hipError_t launch(const pv_dev_cohort& D, const int64_t* wa, const int64_t* ws, 
         // (at Q = 16384 a timed call stays on st: its side streams would join after the windows kernel's end event)
         // (timing with ev_mid brackets the windows kernel alone, so the call then keeps to one order; with ev_end only,
         // the end event follows the whole call and its joins)
-        const Fork* f = (PV_FORK && may_fork && (Cfg<Q>::REGOPS || !ev_mid)) ? fork_of(st, !Cfg<Q>::REGOPS) : nullptr;
+        const Fork* f = (PV_FORK && may_fork && (Cfg<Q>::REGOPS || !ev_mid) && fork_of(st, !Cfg<Q>::REGOPS, sides)) ? &sides : nullptr;
         // the fork and join events are bound to the kernels they follow (the launch's stop event) rather than recorded
         // after them: a recorded event is a packet of its own in the queue, which the queue's next kernel waits behind
         if (f) hipExtLaunchKernelGGL((slot_kernel<Q>), dim3(HL.nlight), dim3(WAVE), 0, st, nullptr, f->fork, 0u, D, wa, ws, W, bpw, nslots, slotbuf, X, HL);
@@ -2852,8 +2908,9 @@ extern "C" int32_t pv_launch_prepare(const pv_dev_cohort* D, int64_t n, int64_t 
     const uint32_t Q = D->Q;
     if (n <= 0 || W <= 0 || W >= (1ll << 31) || !(Q == 1024 || Q == 2048 || Q == 4096 || Q == 16384)) return PV_OK;
     const uint64_t nslots = (uint64_t)n * (((uint64_t)W + Q - 1) / Q + 1);
-    if (PV_FORK && nslots > (Q == 16384 ? SMALL_SLOTS_Q16 : SMALL_SLOTS) && nslots < (1ull << 31))
-        (void)fork_of((hipStream_t)stream, Q == 16384);                  // else: one stream
+    Fork sides{};
+    if (PV_FORK && nslots > (Q == 16384 ? SMALL_SLOTS_Q16 : SMALL_SLOTS) && nslots < (1ull << 31) && !capturing((hipStream_t)stream))
+        (void)fork_of((hipStream_t)stream, Q == 16384, sides);           // else: one stream
     return PV_OK;
 }
 
@@ -3054,7 +3111,7 @@ extern "C" int32_t pv_streams_concurrent(void* a, void* b, int32_t* concurrent, 
     if (!concurrent) { seterr(err, errcap, "null argument"); return PV_EARG; }
     *concurrent = 0;
     bool at_once = false;
-    const hipError_t e = streams_at_once((hipStream_t)a, (hipStream_t)b, at_once);
+    const hipError_t e = streams_at_once((hipStream_t)a, (hipStream_t)b, at_once, true);
     if (e != hipSuccess) { seterr(err, errcap, hipGetErrorString(e)); return PV_EHIP; }
     *concurrent = at_once ? 1 : 0;
     return PV_OK;

@@ -1,6 +1,7 @@
 """Calls from several threads on one stream: a `fetch` or `windows` call passes slot records from one launch to the next
-through a work buffer, so each thread has its own."""
+through a work buffer, so each thread has its own. And no call waits for what its stream has queued."""
 import threading
+import time
 import types
 
 import numpy as np
@@ -112,3 +113,54 @@ def test_noalloc_short_q16k_calls_share_nothing(fx, oracle_ref):
     torch.cuda.synchronize()
     for a, s, W, _, _, out, status in calls:
         assert int(status) == 0 and np.array_equal(out[0].cpu().numpy(), full[a][s:s + W]), (a, s, W)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("ds,n", [("q4k", 8192 + 100), ("q16k", 1024 + 100)])
+def test_first_large_call_on_a_busy_stream_returns(fx, oracle_ref, ds, n):
+    """The first calls on a stream that make side streams return while earlier work still runs there (a spin kernel of
+    about half a second), and the bytes are right; so are those of later calls, which find the stream dry."""
+    import panvram_amd
+    from panvram_amd import _native as N
+    c = panvram_amd.Cohort.open(fx["dirs"][ds], device="cuda", dataset=ds, reference=fx["ref"])
+    L, err, W = N.lib(), N.errbuf(), 300
+    arcs = [O.Archive(f"{fx['dirs'][ds]}/{nm}.{ds}.rr3") for nm in c.names]
+    rng = np.random.default_rng(3)
+    asm = rng.integers(0, len(c), n)
+    start = np.array([rng.integers(0, arcs[a].nbases - W) for a in asm])
+    want = O.windows(arcs, oracle_ref, asm, start, W)
+    ta, ts = torch.from_numpy(asm).cuda(), torch.from_numpy(start).cuda()
+    wb = int(L.pv_windows_work_bytes(c._Dref, n, W))
+    work = [torch.empty(wb, dtype=torch.uint8, device="cuda") for _ in range(2)]
+    out = [torch.empty((n, W), dtype=torch.uint8, device="cuda") for _ in range(6)]
+    status = torch.zeros(1, dtype=torch.int32, device="cuda")
+    warm, busy = torch.cuda.Stream(), torch.cuda.Stream()
+
+    def call(stream, k, w):
+        assert L.pv_windows_hip(c._Dref, ta.data_ptr(), ts.data_ptr(), n, W, None, 0, 1, out[k].data_ptr(), status.data_ptr(),
+                                work[w].data_ptr(), wb, stream.cuda_stream, err, len(err)) == 0, err.value
+
+    torch.cuda.synchronize()
+    call(warm, 0, 0)                                # the kernels are loaded
+    with torch.cuda.stream(busy):
+        torch.cuda._sleep(1000)
+        torch.cuda.synchronize()
+        t = time.perf_counter()
+        torch.cuda._sleep(1_000_000)
+        torch.cuda.synchronize()
+        ticks = int(1_000_000 * 0.5 / (time.perf_counter() - t))
+        torch.cuda._sleep(ticks)
+        done = torch.cuda.Event()
+        done.record()
+    t = time.perf_counter()
+    for k in (1, 2, 3):
+        call(busy, k, 1)
+    took = time.perf_counter() - t
+    assert not done.query() and took < 0.25, took
+    torch.cuda.synchronize()
+    for k in (4, 5):                                # (the stream is dry: the trial is made here)
+        call(busy, k, 1)
+        torch.cuda.synchronize()
+    assert int(status) == 0
+    for x in out:
+        assert np.array_equal(x.cpu().numpy(), want)
