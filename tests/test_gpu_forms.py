@@ -2,7 +2,8 @@
 Cohort.open(packed_reference=, compact_blocks=) holds fewer bytes and returns, byte for byte, what the CPU oracle
 returns at the same coordinates - on the reference's fixtures (q1k, q4k, q16k), on the generated `mini` cohort (soft
 mask, reverse-complemented pieces) and on `wide` (IUPAC runs in the reference, an N run across base 2^22, block
-starts in the compact table's exception list). Run with -m gpu."""
+starts in the compact table's exception list), and on a small reference cut into many pieces (copies off the staged span
+that touch the reference's ends and its runs of other bytes). Run with -m gpu."""
 import os
 
 import numpy as np
@@ -75,3 +76,30 @@ def test_forms_on_generated_cohorts(request, cohort, form):
         assert np.array_equal(np.asarray(c.decode(i)), A.full(ref))
         ok, h = c.check_full(i)
         assert ok and h == c.info(i)["fasta_xxh3"], (i, h)
+
+
+@pytest.mark.parametrize("Q", [1024, 4096, 16384])
+def test_packed_copies_off_the_span(tmp_path, Q):
+    """A 40 kbp reference with a run of IUPAC codes every hundred bases or so, each haplotype cut into pieces of a few
+    hundred bases to a few kbp, half of them reverse-complemented: 16-base reads at the reference's first and last bases and
+    at runs that begin, end or lie inside them, in each kernel that replays (one window, small and large calls, the wave
+    decoder alone). Equal to the oracle."""
+    import panvram_amd
+    from tests import cohortgen as G
+    G.make("mini", str(tmp_path), threads=4, ref={"lengths": [25_000, 15_000], "iupac_runs": 400, "n_runs": 2, "n_run_max": 30},
+           asm={"Q": Q, "n_asm": 6, "frag_min": 12, "frag_max": 60, "sv_per_contig": 1, "sv_max": 200, "seed": 401 + Q})
+    fa = str(tmp_path / "reference.fa")
+    ref = O.reference_bases(fa)
+    full = [O.Archive(str(p)).full(ref) for p in sorted(tmp_path.glob("*.rr3"))]
+    c = panvram_amd.Cohort.open(str(tmp_path), device="cuda", dataset=None, reference=fa, packed_reference=True, compact_blocks=Q != 1024)
+    rng = np.random.default_rng(Q)
+    many = (2048 if Q == 16384 else 16384) // 2 + 500
+    for light in (True, False):
+        c.light_decode = light
+        for a, want in enumerate(full):
+            assert np.array_equal(c.windows(torch.tensor([a]), torch.tensor([0]), len(want))[0].cpu().numpy(), want), (light, a)
+        for n, W in ((1, 300), (300, 1500), (many, 777)):
+            a = rng.integers(0, len(full), n)
+            s = np.array([rng.integers(0, len(full[i]) - W + 1) for i in a])
+            x = c.windows(torch.from_numpy(a).cuda(), torch.from_numpy(s).cuda(), W).cpu().numpy()
+            assert np.array_equal(x, np.stack([full[i][t:t + W] for i, t in zip(a, s)])), (light, n, W)

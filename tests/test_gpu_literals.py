@@ -18,7 +18,7 @@ def _cohort(d, Q, odd, lo, hi, per):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("Q", [1024, 4096, 16384])
+@pytest.mark.parametrize("Q", [1024, 2048, 4096, 16384])
 @pytest.mark.parametrize("odd,lo,hi,per", [(0.0, 9, 60, 300), (0.02, 9, 60, 300), (0.0, 150, 900, 60), (0.002, 150, 900, 60)])
 def test_literal_windows_equal_oracle(tmp_path, Q, odd, lo, hi, per):
     import panvram_amd
