@@ -394,10 +394,15 @@ __device__ __forceinline__ v4u packed16(const RefView& R, uint64_t q) {
     for (; r < R.pne; r++) {
         const uint64_t rs = (uint64_t)R.pes[r], re = rs + (uint64_t)R.pel[r];
         if (rs >= q + 16) break;
-        const uint32_t b = R.peb[r];
+        if (re <= q) continue;
+        // bytes [lo, hi) of the 16: a bit each, spread to a byte mask per dword
+        const uint32_t lo = rs > q ? (uint32_t)(rs - q) : 0u, hi = re < q + 16 ? (uint32_t)(re - q) : 16u;
+        const uint32_t m = (1u << hi) - (1u << lo), b = R.peb[r] * 0x01010101u;
 #pragma unroll
-        for (int i = 0; i < 16; i++)
-            if (q + i >= rs && q + i < re) v[i / 4] = (v[i / 4] & ~(0xFFu << (8 * (i % 4)))) | b << (8 * (i % 4));
+        for (int i = 0; i < 4; i++) {
+            const uint32_t k = ((((m >> (4 * i)) & 15u) * 0x00204081u) & 0x01010101u) * 0xFFu;
+            v[i] = (v[i] & ~k) | (b & k);
+        }
     }
     return v;
 }
@@ -1791,6 +1796,10 @@ __device__ __forceinline__ void process_slot(LS& S, const pv_dev_cohort& D, cons
                 return;
             }
         } else {
+            // (In the packed form a copy off the span goes byte by byte below. Read 16 bases a lane (packed16) it made every
+            // copy of a long block's slot dearer, on the span or off it: windows_kernel on 2^25 bases of a haplotype of 8
+            // SNVs in 1,000 bases 149 us without such a branch, 223 with it, 331 with reverse complements on the span in
+            // it too; the rearranged cohort's light slots take their bases through op16.)
             if (kind == 1 && i1 > i0 + 8 && so < R.wlen && i1 - i0 <= R.wlen - so) {
                 // wholly inside the staged span: aligned destination words, each assembled from two source words
                 const uint32_t a0 = dst + i0, a1 = dst + i1, b0 = (a0 + 3) & ~3u, b1 = a1 & ~3u;
@@ -1801,32 +1810,6 @@ __device__ __forceinline__ void process_slot(LS& S, const pv_dev_cohort& D, cons
                 for (uint32_t q = b0 + 4 * l; q < b1; q += 4 * WAVE) {
                     const uint32_t o = sh + (q - b0);
                     *(uint32_t*)&S.blk[q] = __builtin_amdgcn_alignbyte(rw[(o >> 2) + 1], rw[o >> 2], o & 3);
-                }
-                return;
-            }
-            if (R.pw && (kind & 1) && i1 > i0 + 8) {
-                // off the staged span in the packed form: 16 bytes per lane per pass, the destination's first 16-byte
-                // boundary splitting the head off (a byte per lane at a time, each with its own word, bucket and run
-                // reads, took most of the kernel's time where pieces of the assembly are rearranged)
-                const uint64_t top = (uint64_t)src + len - 1;
-                const uint32_t a0 = dst + i0, a1 = dst + i1, b0 = min((a0 + 15) & ~15u, a1);
-                auto one = [&](uint32_t at) {
-                    S.blk[at] = kind == 1 ? ref_at(S, R, (uint64_t)src + (at - dst)) : pvc::comp(ref_at(S, R, top - (at - dst)));
-                };
-                if (l < b0 - a0) one(a0 + l);
-                for (uint32_t q = b0 + 16 * l; q < a1; q += 16 * WAVE) {
-                    const uint32_t off = q - dst;
-                    if (q + 16 <= a1) {
-                        v4u v = packed16(R, kind == 1 ? (uint64_t)src + off : top - off - 15);
-                        if (kind == 3) {
-                            const v4u u = v;
-                            v.x = comp4(__builtin_bswap32(u.w)); v.y = comp4(__builtin_bswap32(u.z));
-                            v.z = comp4(__builtin_bswap32(u.y)); v.w = comp4(__builtin_bswap32(u.x));
-                        }
-                        *(v4u*)&S.blk[q] = v;
-                    } else {
-                        for (uint32_t i = q; i < a1; i++) one(i);
-                    }
                 }
                 return;
             }
@@ -1926,22 +1909,13 @@ __device__ __forceinline__ void process_slot(LS& S, const pv_dev_cohort& D, cons
             return true;
         } else {
             if (kind == 0) { v = lds16((const uint32_t*)S.aux, src + off); return true; }
-            if (kind == 1) {
-                const uint64_t so = (uint64_t)src + off - (uint64_t)R.wbase;
-                if (!(so < R.wlen && R.wlen - so >= 20)) {
-                    if (!R.pw || (uint64_t)src + off + 16 > R.n) return false;
-                    v = packed16(R, (uint64_t)src + off);
-                    return true;
-                }
-                v = lds16((const uint32_t*)S.refw, (uint32_t)so);
-                return true;
-            }
             const uint64_t top = (uint64_t)src + len - 1;
-            if (top < (uint64_t)off + 15) return false;
-            const uint64_t so = top - off - 15 - (uint64_t)R.wbase;
+            if (kind != 1 && top < (uint64_t)off + 15) return false;
+            const uint64_t q = kind == 1 ? (uint64_t)src + off : top - off - 15, so = q - (uint64_t)R.wbase;
             const bool in = so < R.wlen && R.wlen - so >= 20;
-            if (!in && !R.pw) return false;
-            const v4u u = in ? lds16((const uint32_t*)S.refw, (uint32_t)so) : packed16(R, top - off - 15);
+            if (!in && (!R.pw || q + 16 > R.n)) return false;
+            const v4u u = in ? lds16((const uint32_t*)S.refw, (uint32_t)so) : packed16(R, q);
+            if (kind == 1) { v = u; return true; }
             v.x = comp4(__builtin_bswap32(u.w)); v.y = comp4(__builtin_bswap32(u.z));
             v.z = comp4(__builtin_bswap32(u.y)); v.w = comp4(__builtin_bswap32(u.x));
             return true;

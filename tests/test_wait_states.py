@@ -91,14 +91,22 @@ def violations(lines):
     return found
 
 
-def test_wait_states(tmp_path):
-    tools = [os.path.join(BIN, t) for t in ("llvm-objcopy", "clang-offload-bundler", "llvm-objdump")]
-    if not os.path.exists(LIB) or not all(shutil.which(t) for t in tools):
+def code_object(tmp_path):
+    """The gfx950 code object of the built library, and ROCm's tool by name."""
+    def tool(t):
+        return os.path.join(BIN, t)
+    if not os.path.exists(LIB) or not all(shutil.which(tool(t)) for t in ("llvm-objcopy", "clang-offload-bundler", "llvm-objdump", "llvm-readelf")):
         pytest.skip("needs the built library and ROCm's binary tools")
     fat, co = str(tmp_path / "fat.bin"), str(tmp_path / "k.co")
-    subprocess.run([tools[0], "-O", "binary", "--only-section=.hip_fatbin", LIB, fat], check=True)
-    subprocess.run([tools[1], "--type=o", "--unbundle", f"--input={fat}", "--targets=hipv4-amdgcn-amd-amdhsa--gfx950", f"--output={co}"], check=True)
-    text = subprocess.run([tools[2], "-d", "--no-show-raw-insn", co], check=True, capture_output=True, text=True).stdout
+    subprocess.run([tool("llvm-objcopy"), "-O", "binary", "--only-section=.hip_fatbin", LIB, fat], check=True)
+    subprocess.run([tool("clang-offload-bundler"), "--type=o", "--unbundle", f"--input={fat}", "--targets=hipv4-amdgcn-amd-amdhsa--gfx950",
+                    f"--output={co}"], check=True)
+    return co, tool
+
+
+def test_wait_states(tmp_path):
+    co, tool = code_object(tmp_path)
+    text = subprocess.run([tool("llvm-objdump"), "-d", "--no-show-raw-insn", co], check=True, capture_output=True, text=True).stdout
     lines = text.splitlines()
     assert any("v_cmpx_lt_u32_sdwa" in x for x in lines)                     # the literal loop is there to be checked
     bad = violations(lines)
