@@ -1542,9 +1542,15 @@ template <int Q> constexpr uint64_t small_slots() { return Cfg<Q>::REGOPS ? SMAL
 // ONE: a call of one window of at most 64 slots (a fetch): its light wave stages the window's assembly's model table in
 // LDS (every slot shares it) before its lanes decode, so that the decode's table reads wait on LDS, not on L2 or HBM.
 // Such a call takes this kernel at Q = 16384 too: a fetch of 5,000 bases 93.5 us by the wave decoder in windows_kernel
-// (65 us of it, after a launch for the coordinates) and 71.6 us by a light lane here (46 us) and the replay (13 us).
+// (65 us of it, after a launch for the coordinates) and 71.6 us by a light lane here (46 us) and the replay (13 us). A
+// block over light_pay() bytes (2 in 1,000 of that cohort) has the lookup here ahead of the wave decoder: 3 % more.
+// Four waves per SIMD: where most blocks are long there is a wave at work per slot, and the literal loop's fixed registers
+// otherwise leave 139 VGPRs, three waves (2^25 bases of a haplotype of 8 SNVs in 1,000 bases 422 us, 375 with four; 381
+// with the literal step before that loop, at 126). The heavy kernels of large calls, one wave per 64 slots, run no faster
+// for it (2^28 bases 173.5 us a call, 175.9 with four: two VGPRs go to scratch).
 template <int Q, bool ONE = false>
-__global__ void __launch_bounds__(WAVE) front_kernel(pv_dev_cohort D, const int64_t* __restrict__ wasm, const int64_t* __restrict__ wstart,
+__global__ void __launch_bounds__(WAVE) __attribute__((amdgpu_waves_per_eu(4)))
+front_kernel(pv_dev_cohort D, const int64_t* __restrict__ wasm, const int64_t* __restrict__ wstart,
                                                      uint32_t W, uint32_t bpw, uint64_t nslots, uint8_t* __restrict__ slotbuf, SampleIn X,
                                                      HeavyList HL) {
     if constexpr (Cfg<Q>::REGOPS) {                   // (no heavy role where ops live in LDS: nworkers is 0)

@@ -29,3 +29,10 @@ def test_packed_replay(kernels, Q):
     vgpr, sgpr_spill, vgpr_spill = kernels[f"windows_kernel<{Q}, false, false, false>"]
     assert vgpr <= 64 and sgpr_spill == 0 and vgpr_spill == 0
     assert kernels[f"windows_kernel<{Q}, true, false, false>"][1] <= 256
+
+
+@pytest.mark.parametrize("Q", [1024, 2048, 4096])
+def test_front_kernel_four_waves(kernels, Q):
+    """front_kernel decodes each long block by a wave of its own: 128 VGPRs, four waves per SIMD."""
+    vgpr, _, vgpr_spill = kernels[f"front_kernel<{Q}, false>"]
+    assert vgpr <= 128 and vgpr_spill <= 4
