@@ -201,7 +201,8 @@ typedef struct pv_dev_cohort {
  * Replaces _C.windows_cuda / pv_windows_cuda + run_windows (reference csrc/pv_cuda.cu:117-162), including its checks:
  * Q in {1024, 2048, 4096, 16384}, 0 <= W < 2^31, n * (ceil(W/Q)+1) < 2^31 -> PV_EARG.
  * A call that uses the work buffer refuses a stream under graph capture (PV_EARG): its list and done words carry a
- * number drawn on the host per launch, which a replayed graph would repeat. */
+ * number drawn on the host per launch, which a replayed graph would repeat. At Q = 16384 a call of one or two (window,
+ * covering block) slots (n = 1, W <= 16384) on a stream under capture leaves the buffer alone and may be captured. */
 int32_t pv_windows_hip(const pv_dev_cohort* D, const int64_t* asm_idx, const int64_t* start, int64_t n, int64_t W,
                        const uint8_t* rc, int32_t tokens, int32_t apply_case, uint8_t* out, int32_t* status,
                        void* work, uint64_t work_bytes, void* stream, char* err, size_t errcap);
@@ -254,8 +255,9 @@ int32_t pv_windows_ids_hip(const pv_dev_cohort* D, const int64_t* asm_idx, const
  * host-to-device copies of those tensors and the fill of the status word. `rec` is device memory of 32 bytes, 16-byte
  * aligned: the call's first kernel on `stream` writes the assembly (i64, byte 0), the start (i64, byte 8) and the
  * strand (u8, byte 16; rc != 0 reverse-complements) there and zeroes the int32 status word at byte 24, which the
- * decode then sets as pv_windows_hip's status (with a work buffer below 16 K block size the decode kernel itself,
- * which takes the coordinates as arguments; otherwise a small kernel of its own first). out: u8[W]; apply_case is on. work, errors and the rest as pv_windows_hip with n = 1.
+ * decode then sets as pv_windows_hip's status (with a work buffer the decode kernel itself, which takes the coordinates as
+ * arguments; otherwise, and for a captured call of W <= 16384 at Q = 16384, a small kernel of its own first). out: u8[W];
+ * apply_case is on. work, errors and the rest as pv_windows_hip with n = 1.
  * Consecutive calls may reuse `rec` on one stream (the launches are ordered). No reference counterpart as a C
  * function. */
 int32_t pv_fetch_hip(const pv_dev_cohort* D, int64_t assembly, int64_t start, int64_t W, int32_t rc, int32_t tokens,

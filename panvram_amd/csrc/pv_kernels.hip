@@ -535,7 +535,8 @@ template <int Q, bool G> __device__ __forceinline__ int decode_block(const DecMe
                 }
             } else {
                 // long run: order-2 context on the run's own literals (first: 16, then (previous * 4 + this) & 15).
-                // The first literal takes the general path; then groups of eight literal pairs, then the general path.
+                // The first literal takes the general path; then windows of nine literals (literal_windows), and what is
+                // left of the run the general path again.
                 uint32_t r = 16, j = 0;
                 {
                     const uint32_t s = sym_small(d, SR, SR_LIT2 + 16);
@@ -1477,7 +1478,10 @@ __global__ void __launch_bounds__(WAVE) heavy_kernel(pv_dev_cohort D, const int6
 // LONG: a call of windows of LONG_BPW slots or more (a chromosome, a stream decode), where most waves hold slots of one
 // window and so of one assembly: such a wave stages that model table in LDS first, so that its lanes' table reads wait
 // on LDS instead of L2 (a wave of mixed assemblies reads them from HBM). Its 10 KB per wave would cost the other calls
-// half their waves per CU, and at 16 K block size hold back the whole-slot pass beside this kernel (50 KB per wave).
+// half their waves per CU, and at 16 K block size hold back the whole-slot pass beside this kernel (50 KB per wave). us a
+// call with the table in LDS / without: one window of 2^28 bases 174 / 176 (this kernel 53 / 64), of 2^26 at 1 K blocks
+// 125 / 132 (38 / 46), four of 2^26 175 / 180; windows of 33 to 318 slots within 1.5 % of each other, either way; 65,536
+// windows of three slots, packed reference, 841 / 797.
 constexpr uint32_t LONG_BPW = 256;
 template <int Q, bool LONG>
 __global__ void __launch_bounds__(WAVE) light_decode_kernel(pv_dev_cohort D, const int64_t* __restrict__ wasm, const int64_t* __restrict__ wstart,
