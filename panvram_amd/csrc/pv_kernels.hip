@@ -1806,10 +1806,6 @@ __device__ __forceinline__ void process_slot(LS& S, const pv_dev_cohort& D, cons
                 return;
             }
         } else {
-            // (In the packed form a copy off the span goes byte by byte below. Read 16 bases a lane (packed16) it made every
-            // copy of a long block's slot dearer, on the span or off it: windows_kernel on 2^25 bases of a haplotype of 8
-            // SNVs in 1,000 bases 149 us without such a branch, 223 with it, 331 with reverse complements on the span in
-            // it too; the rearranged cohort's light slots take their bases through op16.)
             if (kind == 1 && i1 > i0 + 8 && so < R.wlen && i1 - i0 <= R.wlen - so) {
                 // wholly inside the staged span: aligned destination words, each assembled from two source words
                 const uint32_t a0 = dst + i0, a1 = dst + i1, b0 = (a0 + 3) & ~3u, b1 = a1 & ~3u;
@@ -1825,6 +1821,22 @@ __device__ __forceinline__ void process_slot(LS& S, const pv_dev_cohort& D, cons
             }
         }
         if (kind == 1) {
+            if constexpr (SPAN) {
+                if (R.pw && i1 > i0 + WAVE) {
+                    // off the staged span in the packed form: 16 bases per lane between the destination's 16-byte
+                    // boundaries, the ends a byte per lane (a byte at a time each takes its own word, bucket and run reads).
+                    // Here, past the copies on the span, and for this strand alone: ahead of both byte loops, for either
+                    // strand, it made every copy of a long block dearer, on the span or off it. windows_kernel, mean (max)
+                    // us without / here / there: sample(1024, 8192) of the human cohort 14.7 (34) / 12.7 (15) / 13.6 (20),
+                    // of a rearranged one 23.2 / 19.3 / 24.3; 2^25 bases of a haplotype of 8 SNVs in 1,000 bases 148 / 151
+                    // / 331.
+                    const uint32_t a0 = dst + i0, a1 = dst + i1, b0 = (a0 + 15) & ~15u, b1 = a1 & ~15u;
+                    for (uint32_t q = b0 + 16 * l; q < b1; q += 16 * WAVE) *(v4u*)&S.blk[q] = packed16(R, (uint64_t)src + (q - dst));
+                    if (l < b0 - a0) S.blk[a0 + l] = ref_at(S, R, (uint64_t)src + i0 + l);
+                    if (l < a1 - b1) S.blk[b1 + l] = ref_at(S, R, (uint64_t)src + (b1 - dst) + l);
+                    return;
+                }
+            }
             // four bytes per lane in flight per pass
             uint32_t i = i0 + l;
             for (; i + 3 * WAVE < i1; i += 4 * WAVE) {

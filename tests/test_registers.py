@@ -25,9 +25,11 @@ def kernels(tmp_path_factory):
 @pytest.mark.parametrize("Q", [1024, 2048, 4096])
 def test_packed_replay(kernels, Q):
     """The replay-only kernel of the packed form keeps its scalars (each spilled one is a lane read in a loop over copies)
-    and the waves its LDS allows; the kernel with the decoder does not spill hundreds for the sake of the packed form."""
+    and the waves its LDS allows; the kernel with the decoder does not spill hundreds for the sake of the packed form.
+    Bounds: 64 VGPRs are eight waves per SIMD, twice what the LDS lets in; with 2 spilled SGPRs the replay of 65,536 windows
+    takes as long as with none (417 us), with 135 it took 426."""
     vgpr, sgpr_spill, vgpr_spill = kernels[f"windows_kernel<{Q}, false, false, false>"]
-    assert vgpr <= 64 and sgpr_spill == 0 and vgpr_spill == 0
+    assert vgpr <= 64 and sgpr_spill <= 16 and vgpr_spill == 0
     assert kernels[f"windows_kernel<{Q}, true, false, false>"][1] <= 256
 
 
