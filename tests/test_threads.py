@@ -164,3 +164,39 @@ def test_first_large_call_on_a_busy_stream_returns(fx, oracle_ref, ds, n):
     assert int(status) == 0
     for x in out:
         assert np.array_equal(x.cpu().numpy(), want)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("ds,n", [("q4k", 8192 + 100), ("q16k", 1024 + 100)])
+def test_large_calls_of_threads_equal_oracle(fx, oracle_ref, ds, n):
+    """Three threads whose large calls share a stream, from the first call on it (one of them tries and replaces the side
+    streams while the others use them), on several streams in turn, so that some share a hardware queue with theirs."""
+    import panvram_amd
+    c = panvram_amd.Cohort.open(fx["dirs"][ds], device="cuda", dataset=ds, reference=fx["ref"])
+    arcs = [O.Archive(f"{fx['dirs'][ds]}/{nm}.{ds}.rr3") for nm in c.names]
+    rng, W, jobs = np.random.default_rng(5), 300, []
+    for _ in range(3):
+        asm = rng.integers(0, len(c), n)
+        start = np.array([rng.integers(0, arcs[a].nbases - W) for a in asm])
+        jobs.append((torch.from_numpy(asm).cuda(), torch.from_numpy(start).cuda(), torch.from_numpy(O.windows(arcs, oracle_ref, asm, start, W)).cuda()))
+    streams = [torch.cuda.Stream() for _ in range(5)]
+    torch.cuda.synchronize()
+    bad, meet = [], threading.Barrier(3)
+
+    def work(t):
+        try:
+            a, s, want = jobs[t]
+            for st in streams:
+                with torch.cuda.stream(st):
+                    meet.wait(60)
+                    for k in range(5):
+                        if not torch.equal(c.windows(a, s, W, check=k % 2 == 0), want):
+                            bad.append((t, k))
+        except Exception as e:
+            bad.append((t, repr(e)))
+            meet.abort()
+
+    ts = [threading.Thread(target=work, args=(t,)) for t in range(3)]
+    [t.start() for t in ts]
+    [t.join() for t in ts]
+    assert not bad, bad[:5]
